@@ -161,8 +161,8 @@ int k2q_gemm_w8a8(const int8_t* qx, const float* sx, const int8_t* qw, const flo
  * codes qx / sx.  Segment i is k2q_gemm_w8a8 of its own weights into its own output y (M x N, row stride N)
  * with its factors u[:, u_col .. u_col + r) (u: M rows of ldu f32, r as for k2q_gemm_w8a8; lora_b NULL: no
  * adapter on that segment); the outputs are bit-identical to nseg separate k2q_gemm_w8a8 calls.
- * 1 <= nseg <= 4, every N a multiple of 256, M > 8.  The launch runs full-K tiles only: ws / ws_bytes are
- * accepted for symmetry with k2q_gemm_w8a8 and not used (pass NULL, 0). */
+ * 1 <= nseg <= 4, every N a multiple of 256, M > 8.  ws: as for k2q_gemm_w8a8 with N the
+ * segments' total (k2q_gemm_w8a8_ws_bytes(M, sum_i N_i, K) bytes; NULL: full-K tiles only, the same result). */
 typedef struct {
   const int8_t* qw;       /* N x K int8 codes */
   const float* sw;        /* N f32 scales */
@@ -293,6 +293,11 @@ typedef struct {
 } k2q_dx_segment;
 int k2q_gemm_dx_grouped(const k2q_dx_segment* seg, int64_t nseg, int64_t M, int64_t K, const float* g, int64_t ldg,
                         const float* lora_a, int64_t r, uint16_t* dx, void* stream);
+/* k2q_gemm_dx_grouped with a workspace for the split schedule (a short last round of tiles over a long reduction is
+ * cut along it, as in k2q_gemm_dx_lin; f32 pieces added in a fixed order): k2q_gemm_dx_ws_bytes(M, sum_i N_i, K)
+ * bytes.  ws NULL or too small: full-reduction tiles only, what k2q_gemm_dx_grouped runs. */
+int k2q_gemm_dx_grouped_ws(const k2q_dx_segment* seg, int64_t nseg, int64_t M, int64_t K, const float* g, int64_t ldg,
+                           const float* lora_a, int64_t r, uint16_t* dx, void* ws, int64_t ws_bytes, void* stream);
 
 
 #ifdef __cplusplus

@@ -93,6 +93,7 @@ _SIGNATURES = {
     "k2q_gemm_dx_ws_bytes": ([_i64, _i64, _i64], _i64),
     "k2q_gemm_dx": ([_p, _p, _i64, _i64, _i64, _p, _p, _i64, _p, _p, _i64, _p], _int),
     "k2q_gemm_dx_grouped": ([_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p], _int),
+    "k2q_gemm_dx_grouped_ws": ([_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p], _int),
 }
 EXPORTS = tuple(_SIGNATURES)
 
@@ -720,8 +721,10 @@ def gemm_w8a8_grouped(qx, sx, segments, u=None):
         keep.extend([qw, sw, bias, lb])
         arr[i] = W8A8Segment(_ptr(qw), _ptr(sw), _ptr(bias), _ptr(lb), _ptr(y), N, int(u_col or 0), float(scale))
     _device_check(dev)
-    _check(load().k2q_gemm_w8a8_grouped(_ptr(qx), _ptr(sx), M, K, ctypes.cast(arr, ctypes.c_void_p), len(segments),
-                                        _ptr(u), r, ldu, None, 0, _stream(dev)), "k2q_gemm_w8a8_grouped")
+    lib = load()
+    ws, nws = _workspace(lib.k2q_gemm_w8a8_ws_bytes(M, sum(o.shape[1] for o in outs), K), dev)
+    _check(lib.k2q_gemm_w8a8_grouped(_ptr(qx), _ptr(sx), M, K, ctypes.cast(arr, ctypes.c_void_p), len(segments),
+                                     _ptr(u), r, ldu, _ptr(ws), nws, _stream(dev)), "k2q_gemm_w8a8_grouped")
     return outs
 
 
@@ -903,8 +906,10 @@ def gemm_dx_grouped(segments, g=None, lora_a=None) -> torch.Tensor:
         _check_rank(r)
     _device_check(dev)
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
-    _check(load().k2q_gemm_dx_grouped(ctypes.addressof(arr), len(segments), M, K, _ptr(g), ldg,
-                                      _ptr(lora_a) if r else None, r, _ptr(dx), _stream(dev)),
+    lib = load()
+    ws, nws = _workspace(lib.k2q_gemm_dx_ws_bytes(M, sum(dy.shape[1] for dy, _ in segments), K), dev)
+    _check(lib.k2q_gemm_dx_grouped_ws(ctypes.addressof(arr), len(segments), M, K, _ptr(g), ldg,
+                                      _ptr(lora_a) if r else None, r, _ptr(dx), _ptr(ws), nws, _stream(dev)),
            "k2q_gemm_dx_grouped")
     return dx
 

@@ -146,6 +146,30 @@ __device__ __forceinline__ v4i frag(const uint8_t* s, int row, int chunk) {
   return *reinterpret_cast<const v4i*>(s + row * BKB + 16 * (chunk ^ swz(row)));
 }
 
+// A grouped forward's segment of A-row A0: its operands, scales, factors and output in p, A0 the row within it.
+template <int NS>
+__device__ __forceinline__ void pick_segment(const GemmArgsN<NS>& p0, GemmBase& p, int64_t& A0) {
+  if (p0.nseg <= 0) return;
+  int s = 0;
+#pragma unroll
+  for (int i = 1; i < NS; ++i) s = (i < p0.nseg && A0 >= p0.seg[i].start) ? i : s;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    if (i != s) continue;
+    const GemmSeg& g = p0.seg[i];
+    p.a = g.a;
+    p.sw = g.sw;
+    p.bias = g.bias;
+    p.lora_ra = g.lora_ra;
+    p.lora_rb = g.lora_ra ? p0.lora_rb + g.rb_off : nullptr;
+    p.lora_scale = g.lora_scale;
+    p.out = g.out;
+    p.rows_a = g.rows;
+    p.ldo = g.ldo;
+    A0 -= g.start;
+  }
+}
+
 template <bool BF16, class AccT>
 __device__ __forceinline__ void mma(v4i a, v4i b, AccT& c) {
   if constexpr (std::is_same_v<AccT, v4i>) {   // int8, 16 x 16 blocks
@@ -237,7 +261,7 @@ __device__ __forceinline__ void fwht128_rows(v16f (&f)[4], int h) {
 // lines, paired half lines and whole lines move 24, 31 and 35 B/clk/CU.  A stage is consumed after every
 // wave's `s_waitcnt vmcnt` for it plus one lds_barrier() (the wave's LDS operations, then s_barrier; not
 // __syncthreads, whose full memory fence would drain the prefetches).
-constexpr int SBK = 64;                   // unit of reduction lengths in the split plan (half a stage)
+constexpr int SBK = 64;                   // unit of a piece's reduction range (half a stage)
 constexpr int K2Q_DMA_CPOL = 1;           // cache policy bits of the main-loop copies: sc0
 constexpr int WBK = 128;                  // reduction bytes per stage
 
@@ -321,15 +345,15 @@ __device__ __forceinline__ void wait_vmcnt() {
 // to it); outstanding global loads, the LDS-DMA prefetches among them, are not waited for.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-enum { MODE_TILE = 0, MODE_PIECE = 1, MODE_FIXUP = 2, MODE_KSEG = 3 };
+enum { MODE_TILE = 0, MODE_PIECE = 1, MODE_KPIECE = 2, MODE_KSEG = 3 };
 
 // MODE_TILE: full-K tiles 0 .. dp_tiles-1 with their epilogues; workgroup b takes tiles r * nwg + b'
 // (b' its XCD-remapped id) for rounds r = 0, 1, ... while they exist, so the launch can use fewer
 // workgroups than CUs and give each the same number of tiles.  MODE_PIECE: one piece of a remainder tile,
-// accumulators parked in part.  MODE_FIXUP: the pieces of remainder tile dp_tiles + blockIdx.x added in
-// slice order, then the epilogue.  MODE_KSEG: MODE_TILE over a segmented reduction (the grouped input
-// gradient: the operand pair changes at segment boundaries).  Separate kernels, so the register allocation of
-// the tile kernel is not shared with the other paths.  The split modes run T256 tiles only.
+// accumulators parked in part (gemm_fixup_kernel adds them and runs the epilogue).  MODE_KSEG, MODE_KPIECE: the
+// same two over a segmented reduction (the grouped input gradient: the operand pair changes at segment
+// boundaries).  Separate kernels, so the register allocation of the tile kernel is not shared with the other
+// paths.  The split modes run T256 and T128 tiles only.
 template <int EPI, int MODE, class C, int NS>
 __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p, int64_t lid, int kbeg, int nk);
 
@@ -337,9 +361,7 @@ template <int EPI, int MODE, class C, int NS>
 __global__ __launch_bounds__(GT, C::WPC) __attribute__((amdgpu_waves_per_eu(2 * C::WPC, 2 * C::WPC)))
 void gemm_nt_kernel(GemmArgsN<NS> p) {
   const int64_t nk_full = p.kbytes / SBK;
-  if constexpr (MODE == MODE_FIXUP) {
-    gemm_tile<EPI, MODE, C, NS>(p, p.dp_tiles + blockIdx.x, 0, (int)nk_full);
-  } else if constexpr (MODE == MODE_PIECE) {   // pieces cover whole stage pairs
+  if constexpr (MODE == MODE_PIECE || MODE == MODE_KPIECE) {   // pieces cover whole stage pairs
     const int sl = (int)blockIdx.x / p.sk_rem;
     const int np = (int)(nk_full / 2);
     const int kbeg = 2 * (sl * np / p.sk_s);
@@ -354,8 +376,8 @@ void gemm_nt_kernel(GemmArgsN<NS> p) {
   }
 }
 
-// One output tile (linear id lid) over reduction stages kbeg .. kbeg+nk-1, then its epilogue (MODE_TILE,
-// MODE_FIXUP) or its parked accumulators (MODE_PIECE).
+// One output tile (linear id lid) over reduction stages kbeg .. kbeg+nk-1, then its epilogue (MODE_TILE, MODE_KSEG)
+// or its parked accumulators (MODE_PIECE, MODE_KPIECE).
 template <int EPI, int MODE, class C, int NS>
 __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, int kbeg, int nk) {
   constexpr bool BF16 = (EPI == EPI_DX || EPI == EPI_LIN || EPI == EPI_DXLIN);
@@ -384,31 +406,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
   const int64_t B0 = tb * TB;
   // A grouped forward: the tile's segment supplies the operands (workgroup-uniform, scalar registers); A0
   // becomes the row within the segment.  Constant segment indices keep every field a plain argument load.
-  // Grouped launches run full-K tiles only (no split pieces), so the piece and fixup kernels, at their
-  // register limit, carry none of this.  Segments start on multiples of TA (the launch checks it).
+  // Segments start on multiples of TA (the launch checks it).
   GemmBase p = p0;
-  if constexpr (EPI == EPI_W8 && MODE == MODE_TILE && NS > 0) {
-    if (p0.nseg > 0) {
-      int s = 0;
-#pragma unroll
-      for (int i = 1; i < MAX_SEG; ++i) s = (i < p0.nseg && A0 >= p0.seg[i].start) ? i : s;
-#pragma unroll
-      for (int i = 0; i < MAX_SEG; ++i) {
-        if (i != s) continue;
-        const GemmSeg& g = p0.seg[i];
-        p.a = g.a;
-        p.sw = g.sw;
-        p.bias = g.bias;
-        p.lora_ra = g.lora_ra;
-        p.lora_rb = g.lora_ra ? p0.lora_rb + g.rb_off : nullptr;
-        p.lora_scale = g.lora_scale;
-        p.out = g.out;
-        p.rows_a = g.rows;
-        p.ldo = g.ldo;
-        A0 -= g.start;
-      }
-    }
-  }
+  if constexpr (EPI == EPI_W8 && NS > 0) pick_segment(p0, p, A0);
 
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -461,13 +461,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
     ldb_s = __builtin_amdgcn_readfirstlane((int)ldb);
     const int64_t na = p.rows_a - A0 < TA ? p.rows_a - A0 : TA;
     const int64_t nb = p.rows_b - B0 < TB ? p.rows_b - B0 : TB;
-    rsa = k2q_rsrc(a + A0 * lda + (int64_t)kbeg * SBK, na * lda - (int64_t)kbeg * SBK);
-    rsb = k2q_rsrc(b + B0 * ldb + (int64_t)kbeg * SBK, nb * ldb - (int64_t)kbeg * SBK);
+    const int64_t kb = MODE == MODE_KPIECE ? 0 : (int64_t)kbeg * SBK;   // kbase holds a segmented piece's start
+    rsa = k2q_rsrc(a + A0 * lda + kb, na * lda - kb);
+    rsb = k2q_rsrc(b + B0 * ldb + kb, nb * ldb - kb);
   };
   // Segmented reduction (full-K tiles of EPI_DXLIN only): stage st of segment j reads its operands at stage
   // st - kbase; seek(st) moves to st's segment.  The stages passed to seek increase by at most one per call
   // and every segment holds at least one stage, so one step per call reaches it.
-  constexpr bool KSEGS = (MODE == MODE_KSEG);
+  // A piece's stages count from its first one, s0 of the whole reduction: the segment tables are moved by s0.
+  constexpr bool KSEGS = (MODE == MODE_KSEG || MODE == MODE_KPIECE);
+  const int s0 = MODE == MODE_KPIECE ? kbeg / 2 : 0;
   int kseg = 0, kbase = 0, kend = 0x7fffffff;
   auto bind_seg = [&](int j) {   // j is workgroup-uniform; constant indices keep the fields argument loads
     if constexpr (NS > 0) {
@@ -475,11 +478,20 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
 #pragma unroll
       for (int i = 1; i < NS; ++i) sp = j == i ? &p0.ks[i] : sp;
       bind(sp->a, sp->b, sp->lda_b, sp->ldb_b);
-      kend = sp->end;
+      kend = sp->end - s0;
     }
   };
   if constexpr (KSEGS && NS > 0) {
-    if (p0.nks > 0) bind_seg(0);
+    if constexpr (MODE == MODE_KPIECE) {   // the segment that holds stage s0
+#pragma unroll
+      for (int i = 1; i < NS; ++i)
+        if (i < p0.nks && s0 >= p0.ks[i - 1].end) {
+          kseg = i;
+          kbase = p0.ks[i - 1].end;
+        }
+      kbase -= s0;
+    }
+    if (p0.nks > 0) bind_seg(kseg);
     else bind(p.a, p.b, p.lda_b, p.ldb_b);
   } else {
     bind(p.a, p.b, p.lda_b, p.ldb_b);
@@ -551,32 +563,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
   // workgroup-uniform (scalar registers) and the thread offset a 32-bit vector register.
   constexpr int64_t PIECE_BYTES = (int64_t)TA * TB * 4;
   const uint32_t toff = 16u * tid;
-  if constexpr (MODE == MODE_FIXUP) {
-    for (int sl = 0; sl < p.sk_s; ++sl) {
-      const uint8_t* pc = reinterpret_cast<const uint8_t*>(p.part) + ((int64_t)sl * p.sk_rem + blockIdx.x) * PIECE_BYTES;
-#pragma unroll
-      for (int ia = 0; ia < NA; ++ia)
-#pragma unroll
-        for (int ib = 0; ib < NB; ++ib) {
-          if constexpr (MB == 16) {   // one 16-byte unit per block
-            acc[ia][ib] += *reinterpret_cast<const v4i*>(pc + (int64_t)(ia * NB + ib) * GT * 16 + toff);
-          } else {
-            const uint8_t* u = pc + (int64_t)(ia * NB + ib) * 4 * GT * 16;
-            const v4i q0 = *reinterpret_cast<const v4i*>(u + toff);
-            const v4i q1 = *reinterpret_cast<const v4i*>(u + GT * 16 + toff);
-            const v4i q2 = *reinterpret_cast<const v4i*>(u + 2 * GT * 16 + toff);
-            const v4i q3 = *reinterpret_cast<const v4i*>(u + 3 * GT * 16 + toff);
-            const v16i v = __builtin_shufflevector(__builtin_shufflevector(q0, q1, 0, 1, 2, 3, 4, 5, 6, 7),
-                                                   __builtin_shufflevector(q2, q3, 0, 1, 2, 3, 4, 5, 6, 7), 0, 1,
-                                                   2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-            if constexpr (BF16)
-              acc[ia][ib] = __builtin_bit_cast(v16i, __builtin_bit_cast(v16f, acc[ia][ib]) + __builtin_bit_cast(v16f, v));
-            else
-              acc[ia][ib] += v;
-          }
-        }
-    }
-  } else if constexpr (MB == 16) {
+  if constexpr (MB == 16) {
     // int8 main loop on 16 x 16 blocks.  A stage is two 64-byte windows; a window is a grid of NA x NB
     // v_mfma_i32_16x16x64_i8 (a lane's fragment: 16 bytes of one row, row c16 of the block, chunk 4 w + q4 of
     // window w).  The operand with fewer blocks per wave is "held" (all NH fragments of a window in
@@ -753,7 +740,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
     }
     wait_vmcnt<0>();   // no LDS-DMA may still be in flight when the workgroup's LDS is released
   }
-  if constexpr (MODE == MODE_PIECE) {   // park the accumulators for the fixup launch
+  if constexpr (MODE == MODE_PIECE || MODE == MODE_KPIECE) {   // park the accumulators for the fixup launch
     uint8_t* dst = reinterpret_cast<uint8_t*>(p.part) + (int64_t)blockIdx.x * PIECE_BYTES;
 #pragma unroll
     for (int ia = 0; ia < NA; ++ia)
@@ -1029,6 +1016,173 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
 }
 
 // ---------------------------------------------------------------------------------------------------------
+// The fixup of a split launch: the pieces of each remainder tile added in slice order, then the tile kernel's
+// epilogue on the sums, element for element the same arithmetic (so W8 outputs equal the unsplit launch's bit for
+// bit).  Bound by reading the pieces (s x 256 KB a T256 tile): 72 tiles of 3 pieces (57 MB) take 14.6 us for the
+// input gradient and 18.7 us for W8A8.  A wave owns one column of 32 x 32 blocks (the NA blocks a tile-kernel wave
+// holds for one of its B-blocks: 32 output rows x ARW columns), FIX_WAVES waves a workgroup, so the launches that
+// split (48-128 tiles) spread over every CU; a workgroup per tile, as part of the tile kernel, took 19.5 us for the
+// same W8A8 pieces and knew no segments.  Two slices in flight per wave (registers) and tiles fixed up on the XCD
+// that ran their pieces were 0-37 % slower.  The LoRA factors come straight from global memory, the next 16-rank
+// chunk's loads in flight while this one is multiplied; the bf16 block goes through the wave's own LDS for
+// row-contiguous stores.
+// ---------------------------------------------------------------------------------------------------------
+constexpr int FIX_WAVES = 2;
+template <class C>
+constexpr int fix_wgs_per_tile() { return GW * C::NB / FIX_WAVES; }
+
+template <int EPI, class C, int NS>
+__global__ __launch_bounds__(64 * FIX_WAVES) void gemm_fixup_kernel(GemmArgsN<NS> p0) {
+  constexpr bool BF16 = (EPI == EPI_DX || EPI == EPI_LIN || EPI == EPI_DXLIN);
+  constexpr bool SCALED = (EPI == EPI_W8 || EPI == EPI_LIN);
+  constexpr bool RA_T = (EPI == EPI_DX || EPI == EPI_DXLIN);
+  constexpr int NA = C::NA, NB = C::NB, PER = fix_wgs_per_tile<C>();
+  constexpr int CROW = 2 * C::ARW + 16;
+  __shared__ __attribute__((aligned(16))) uint8_t ctiles[FIX_WAVES][32 * CROW];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int rt = (int)blockIdx.x / PER;                               // remainder tile
+  const int job = ((int)blockIdx.x % PER) * FIX_WAVES + wave;         // tile-kernel wave, and its B-block
+  const int w = job / NB, ib = job % NB;
+  const int wa = w % C::WVA, wb = w / C::WVA;
+  const int h = lane >> 5, c32 = lane & 31;
+
+  const int64_t tiles_a = (p0.rows_a + C::TA - 1) / C::TA, tiles_b = (p0.rows_b + C::TB - 1) / C::TB;
+  int64_t ta, tb;
+  group_coords(p0.dp_tiles + rt, tiles_a, tiles_b, p0.gb > 0 ? p0.gb : 8, ta, tb);
+  int64_t A0 = ta * C::TA;
+  GemmBase p = p0;
+  if constexpr (EPI == EPI_W8 && NS > 0) pick_segment(p0, p, A0);
+  const int64_t a0 = A0 + C::ARW * wa, b0 = tb * C::TB + C::BRW * wb + 32 * ib;
+  if (a0 >= p.rows_a || b0 >= p.rows_b) return;   // no barriers below: a wave past the matrix leaves
+
+  const int64_t rb = b0 + c32 < p.rows_b ? b0 + c32 : p.rows_b - 1;   // this lane's B-row
+  // the first chunk of LoRA factors is on its way under the pieces
+  const bool lora = EPI != EPI_ACC && p.lora_rb != nullptr && p.r > 0;
+  v4f fa[NA][2], fb[2];
+  auto load_factors = [&](int c0) {
+    const float* q = p.lora_rb + rb * p.ldr + c0 + 8 * h;
+    fb[0] = *reinterpret_cast<const v4f*>(q);
+    fb[1] = *reinterpret_cast<const v4f*>(q + 4);
+    if constexpr (EPI == EPI_W8) {
+      for (int i = 1; i < p.rb_parts; ++i) {   // ((part 0 + part 1) + part 2) ..., as the tile kernel adds them
+        fb[0] += *reinterpret_cast<const v4f*>(q + i * p.rb_pstride);
+        fb[1] += *reinterpret_cast<const v4f*>(q + i * p.rb_pstride + 4);
+      }
+    }
+#pragma unroll
+    for (int ia = 0; ia < NA; ++ia) {
+      int64_t ra = a0 + 32 * ia + c32;
+      ra = ra < p.rows_a ? ra : p.rows_a - 1;
+      if constexpr (RA_T) {
+        const float* f = p.lora_ra + (int64_t)(c0 + 8 * h) * p.rows_a + ra;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) fa[ia][j >> 2][j & 3] = f[(int64_t)j * p.rows_a];
+      } else {
+        const float* f = p.lora_ra + ra * p.r + c0 + 8 * h;
+        fa[ia][0] = *reinterpret_cast<const v4f*>(f);
+        fa[ia][1] = *reinterpret_cast<const v4f*>(f + 4);
+      }
+    }
+  };
+
+  using Acc = std::conditional_t<BF16, v16f, v16i>;
+  Acc acc[NA];
+#pragma unroll
+  for (int ia = 0; ia < NA; ++ia) acc[ia] = Acc{0};
+  constexpr int64_t PIECE_BYTES = (int64_t)C::TA * C::TB * 4;
+  const uint32_t toff = 16u * (uint32_t)(64 * w + lane);
+  if (lora) load_factors(0);
+  for (int sl = 0; sl < p.sk_s; ++sl) {
+    const uint8_t* pc = reinterpret_cast<const uint8_t*>(p.part) + ((int64_t)sl * p.sk_rem + rt) * PIECE_BYTES;
+    v4i q[NA][4];
+#pragma unroll
+    for (int ia = 0; ia < NA; ++ia)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        q[ia][j] = *reinterpret_cast<const v4i*>(pc + (int64_t)((ia * NB + ib) * 4 + j) * GT * 16 + toff);
+#pragma unroll
+    for (int ia = 0; ia < NA; ++ia) {
+      const v16i v = __builtin_shufflevector(__builtin_shufflevector(q[ia][0], q[ia][1], 0, 1, 2, 3, 4, 5, 6, 7),
+                                             __builtin_shufflevector(q[ia][2], q[ia][3], 0, 1, 2, 3, 4, 5, 6, 7), 0, 1,
+                                             2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+      acc[ia] += __builtin_bit_cast(Acc, v);
+    }
+  }
+
+  if constexpr (EPI == EPI_ACC) {
+    int32_t* out = static_cast<int32_t*>(p.out);
+    if (b0 + c32 >= p.rows_b) return;
+#pragma unroll
+    for (int ia = 0; ia < NA; ++ia)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t n = a0 + 32 * ia + 8 * j + 4 * h;
+        if (n < p.rows_a)
+          *reinterpret_cast<v4i*>(out + (b0 + c32) * p.ldo + n) =
+              v4i{acc[ia][4 * j], acc[ia][4 * j + 1], acc[ia][4 * j + 2], acc[ia][4 * j + 3]};
+      }
+    return;
+  } else {
+    v16f f[NA];
+    if constexpr (SCALED) {
+      const float sxm = EPI == EPI_W8 ? p.sx[rb] * 0.0078125f : 1.f;
+#pragma unroll
+      for (int ia = 0; ia < NA; ++ia) {
+        v16f a;
+        if constexpr (BF16) a = acc[ia];
+        else a = __builtin_convertvector(acc[ia], v16f);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          int64_t n = a0 + 32 * ia + 8 * j + 4 * h;   // rows_a % 4 == 0: four rows are in the matrix or out of it
+          n = n < p.rows_a ? n : 0;
+          const v4f sw = EPI == EPI_W8 ? *reinterpret_cast<const v4f*>(p.sw + n) : v4f{1.f, 1.f, 1.f, 1.f};
+          const v4f bi = p.bias ? *reinterpret_cast<const v4f*>(p.bias + n) : v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) f[ia][4 * j + i] = __builtin_fmaf(a[4 * j + i], sxm * sw[i], bi[i]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int ia = 0; ia < NA; ++ia) f[ia] = acc[ia];
+      if constexpr (EPI == EPI_DX) fwht128_rows(f, h);
+    }
+    if (lora) {
+      for (int c0 = 0; c0 < p.r; c0 += 16) {
+        v8bf ba[NA];
+#pragma unroll
+        for (int ia = 0; ia < NA; ++ia) ba[ia] = f32x8_to_bf16v(fa[ia][0], fa[ia][1], 1.f);
+        const v8bf bb = f32x8_to_bf16v(fb[0], fb[1], p.lora_scale);
+        if (c0 + 16 < p.r) load_factors(c0 + 16);
+#pragma unroll
+        for (int ia = 0; ia < NA; ++ia) f[ia] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ba[ia], bb, f[ia], 0, 0, 0);
+      }
+    }
+    uint8_t* ct = ctiles[wave];   // this wave's alone: its own LDS operations complete in order
+#pragma unroll
+    for (int ia = 0; ia < NA; ++ia) ctile_put<CROW>(ct, 0, 32 * ia, lane, f[ia]);
+    uint16_t* out = static_cast<uint16_t*>(p.out);
+    constexpr int CPR = C::ARW / 8, RPI = 64 / CPR;   // 16-byte chunks per row, rows per store instruction
+    const int chunk = lane % CPR;
+    const int64_t col = a0 + 8 * chunk;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int row = RPI * i + lane / CPR;
+      const v4u v = *reinterpret_cast<const v4u*>(ct + row * CROW + 16 * chunk);
+      if (b0 + row >= p.rows_b || col >= p.rows_a) continue;
+      uint16_t* o = out + (b0 + row) * p.ldo + col;
+      if ((p.ldo & 7) == 0) {
+        __builtin_nontemporal_store(v, reinterpret_cast<v4u*>(o));
+      } else {                     // ragged widths: element stores
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (col + e < p.rows_a) o[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------
 // W4A8: A operand = packed int4 weights (rows n, K/2 bytes per row), bf16 group scales sw4[g][n].
 // Tile 128 (n) x 128 (m) per 256-thread workgroup, three workgroups per CU (166 VGPRs) so that one wave's
 // per-group scaling runs while another's MFMAs do (wave priority follows the work left, see step()).
@@ -1269,124 +1423,92 @@ int launch_w4(const W4Args& p, hipStream_t st) {
   return k2q_launch_status();
 }
 
-// Split plan for the tiles of the last, partly filled round of T256 tiles, in units of one reduction stage of
-// one tile (measured on MI355X): a full-K tile costs nk + 8 (epilogue); cutting the rem remainder tiles into s
-// pieces (one round of pieces when rem * s <= CUs) costs nk / s per piece plus ~12 (ramp and piece store),
-// and the fixup launch ~20 + 3 per piece read back.  The s with the lowest cost is taken if it saves at least
-// 10 %.
+// Launch plans.  A launch's time is estimated per tile shape, in microseconds, and the cheapest plan taken:
+//   launch + rounds x (stages x stage cost + epilogue),
+// a round being CUs x workgroups-per-CU tiles, and the last, partly filled round (its tiles the remainder) either
+// run like the others or cut along the reduction into s pieces per tile, whose accumulators a fixup launch adds:
+//   ceil(stages / s) x stage cost + piece cost + 0.207 us per MB of pieces.
+// A stage (128 reduction bytes) of a partly filled round is cheaper (less contention for L2 and HBM, and a higher
+// clock), and dearer the more of the staged bytes no other tile shares: its cost is scaled by (alpha + (1 - alpha)
+// fill) (1 + m unique), unique = the operands' rows over the rows that the tiles stage.  The constants are fitted
+// to the measured times of every shape and split at 252 launches (int8 and bf16, M 96-4608, outputs 1536-32768,
+// reductions 1024-32768): the plan taken is on average 1.1 % from the fastest measured one, where the estimate it
+// replaced, fitted to full rounds, was 3.8 % (and 20-38 % on one-round launches of 256 x 256 tiles and on long
+// reductions over few tiles: the 768-token input gradient to 16384 columns 196.6 -> 164.8 us, 512 x 6144 over 16384
+// 157.4 -> 114.0).
 struct SplitPlan {
-  int64_t dp_tiles;
-  int rem, s;
-  double cost;   // stage units of a T256 tile
+  int64_t dp_tiles;   // tiles run over the full reduction
+  int rem, s;         // remainder tiles and their pieces
+  double cost;        // microseconds
 };
 
-SplitPlan split_plan(int64_t tiles, int nk, int cus) {
-  SplitPlan q{tiles, 0, 1, 0.0};
-  const int64_t full = tiles / cus, rem = tiles - full * cus;
-  const double tile = nk + 8.0;
-  q.cost = (double)((tiles + cus - 1) / cus) * tile;
-  if (rem == 0) return q;
-  double best = 0.9 * q.cost;
-  for (int s = 2; s <= 8 && rem * s <= cus && nk / s >= 8; ++s) {
-    const double t = (double)full * tile + (double)nk / s + 12.0 + 20.0 + 3.0 * s;
-    if (t < best) {
-      best = t;
-      q.s = s;
+struct TileCost {
+  int ta, tb, wpc;
+  double alone, shared;   // a stage with one workgroup on a CU, with all its workgroups
+  double epi, piece;      // epilogue; piece ramp and store, fixup launch (0: the shape does not split)
+};
+constexpr TileCost TILE_COSTS[TILE_COUNT] = {
+    {256, 256, 1, 1.466, 1.466, 6.694, 10.84},
+    {256, 320, 1, 1.663, 1.663, 10.847, 0.0},
+    {192, 256, 1, 1.203, 1.203, 5.598, 0.0},
+    {128, 128, 2, 0.605, 0.989, 5.438, 9.167},
+};
+
+// Shortest segmented reduction that is cut (stages).  Below it a launch takes under 60 us and a cut gains a few.
+constexpr int KSEG_SPLIT_MIN = 48;
+
+// The best plan of tile shape t for rows_a x rows_b outputs over nst stages.
+SplitPlan tile_plan(int t, bool bf16, int64_t rows_a, int64_t rows_b, int nst, int cus, bool can_split) {
+  const TileCost& c = TILE_COSTS[t];
+  const int64_t tiles = ((rows_a + c.ta - 1) / c.ta) * ((rows_b + c.tb - 1) / c.tb);
+  const int64_t slots = (int64_t)cus * c.wpc, full = tiles / slots, rem = tiles - full * slots;
+  const double unique = (double)(rows_a + rows_b) / ((double)tiles * (c.ta + c.tb));
+  const double k = (bf16 ? 1.074 : 1.0) * (1.0 + 0.63 * unique), epi = c.epi * (bf16 ? 0.711 : 1.0);
+  auto stage = [&](int64_t active) {
+    if (active > cus) return k * (c.alone + (c.shared - c.alone) * (double)(active - cus) / (double)cus);
+    return k * c.alone * (0.582 + 0.418 * (double)active / (double)cus);
+  };
+  const double head = 1.069 + (double)full * (nst * stage(slots) + epi);
+  SplitPlan q{tiles, 0, 1, head + (rem ? nst * stage(rem) + epi : 0.0)};
+  if (can_split && c.piece > 0.0 && rem > 0) {
+    for (int s = 2; s <= 10 && rem * s <= slots && nst / s >= 4; ++s) {
+      const double mb = (double)(rem * s) * c.ta * c.tb * 4e-6;
+      const double t_s = head + (double)((nst + s - 1) / s) * stage(rem * s) + c.piece + 0.207 * mb;
+      if (t_s < q.cost) q = SplitPlan{full * slots, (int)rem, s, t_s};
     }
   }
-  if (q.s > 1) {
-    q.dp_tiles = full * cus;
-    q.rem = (int)rem;
-    q.cost = best;
-  }
+  // no plan is faster than reading the operands once (5 TB/s)
+  const double floor_us = 3.069 + (double)(rows_a + rows_b) * nst * WBK / 5e6;
+  if (q.cost < floor_us) q.cost = floor_us;
   return q;
 }
 
-// Split plan for a launch of 128 x 128 tiles (two workgroups per CU) that fits one round of workgroup slots:
-// every tile cut along K into s pieces (whole stage pairs), then one fixup launch, when that is estimated at
-// least 5 % faster.  Estimates in microseconds, fitted to MI355X timings of 11 launch shapes (M 256-2048,
-// N 1024-6144, K 3072-16384; split or not, the plan's pick is within 6 % of the fastest measured): a full-K tile
-// 0.62 per 128-byte stage + 6; s pieces 0.62 per stage of the longest piece, x 1.25 once pieces outnumber the
-// CUs, + 10 + 0.035 per piece (piece stores and the fixup).  Long reductions over few tiles gain most: M = 1024,
-// N = 3072, K = 12288 (cfg4's text-stream down projection) 70.5 -> 62.8 us with s = 2.
-SplitPlan split_plan128(int64_t tiles, int nk, int cus) {
-  SplitPlan q{tiles, 0, 1, 0.0};
-  const int64_t slots = 2 * (int64_t)cus;
-  if (tiles > slots) return q;
-  const int np = nk / 2;   // 128-byte stages
-  auto stages_us = [&](int stages, int64_t wgs) { return 0.62 * stages * (wgs > cus ? 1.25 : 1.0); };
-  q.cost = stages_us(np, tiles) + 6.0;
-  double best = 0.95 * q.cost;
-  for (int s = 2; s <= 8 && tiles * s <= slots && np / s >= 4; ++s) {
-    const double t = stages_us((np + s - 1) / s, tiles * s) + 10.0 + 0.035 * (double)(tiles * s);
-    if (t < best) {
-      best = t;
-      q.s = s;
-    }
-  }
-  if (q.s > 1) {
-    q.dp_tiles = 0;
-    q.rem = (int)tiles;
-    q.cost = best;
-  }
-  return q;
-}
-
-// Tile shape of a launch: the one with the lowest estimated time, in units of one reduction stage of a T256 tile.
-// A round of `active` tiles over `slots` = CUs x workgroups-per-CU costs nk x c x (0.7 + 0.3 active / slots) +
-// epilogue: a partly filled round runs its stages faster (less HBM and L2 contention).  Per-stage costs relative
-// to T256, fitted to the MI355X timings of 17 launch shapes (M 1024..16896, N 1536..16384, K 3072..16384; the
-// fitted model picks the fastest measured shape on each): T320 1.25, T192 0.80, T128 0.60 with two workgroups
-// sharing a CU and 0.30 with a CU to itself; epilogues 8 (T256, T320), 7 (T192), 4 (T128).  T256 may instead cut
-// its last round's tiles along K (split_plan), and a launch of T128 tiles its one round (split_plan128).  The
-// rotating input-gradient epilogue runs 128 A-rows per wave (T256 only); grouped launches need segments on tile
-// boundaries (TA = 256 or 128).
 struct TileChoice {
   int tile;
-  SplitPlan split;   // T256 and T128
+  SplitPlan split;   // s > 1 for T256 and T128 only
 };
 
-template <class C>
-double tile_cost(int64_t rows_a, int64_t rows_b, int nk, int cus, double stage_cost, double alone_cost, double epi) {
-  const int64_t tiles = ((rows_a + C::TA - 1) / C::TA) * ((rows_b + C::TB - 1) / C::TB);
-  const int64_t slots = (int64_t)cus * C::WPC;
-  const int64_t full = tiles / slots, rem = tiles - full * slots;
-  auto round = [&](int64_t active) {
-    const double c = (C::WPC > 1 && active <= cus) ? alone_cost : stage_cost;
-    return nk * c * (0.7 + 0.3 * (double)active / (double)slots) + epi;
-  };
-  return (double)full * round(slots) + (rem ? round(rem) : 0.0);
-}
+bool epi_bf16(int epi) { return epi == EPI_DX || epi == EPI_LIN || epi == EPI_DXLIN; }
 
-// allowed: bit t set = tile shape t may be chosen; can_split: T256 may cut its last round along K.
+// allowed: bit t set = tile shape t may be chosen; can_split: the last round may be cut along the reduction.  The
+// rotating input-gradient epilogue runs 128 A-rows per wave (T256 only); grouped launches need segments on tile
+// boundaries (TA = 256 or 128).
 TileChoice choose_tile(int epi, int64_t rows_a, int64_t rows_b, int64_t kbytes, unsigned allowed, bool can_split,
                        int forced, int cus) {
-  const int nk = (int)(kbytes / SBK);
-  const int64_t tiles256 = ((rows_a + 255) / 256) * ((rows_b + 255) / 256);
-  TileChoice c{TILE_256, can_split ? split_plan(tiles256, nk, cus) : SplitPlan{tiles256, 0, 1, 0.0}};
-  const int64_t tiles128 = ((rows_a + 127) / 128) * ((rows_b + 127) / 128);
-  if (forced >= 0) {
-    c.tile = forced;
-    if (forced != TILE_256) c.split = SplitPlan{0, 0, 1, 0.0};
-    if (forced == TILE_128 && can_split) c.split = split_plan128(tiles128, nk, cus);
-    return c;
+  const int nst = (int)(kbytes / WBK);
+  const bool bf16 = epi_bf16(epi);
+  if (epi == EPI_DX) forced = TILE_256;
+  TileChoice best{-1, SplitPlan{0, 0, 1, 0.0}};
+  for (int t = 0; t < TILE_COUNT; ++t) {
+    if (forced >= 0 ? t != forced : !(allowed >> t & 1)) continue;
+    const SplitPlan q = tile_plan(t, bf16, rows_a, rows_b, nst, cus, can_split);
+    if (best.tile < 0 || q.cost < best.split.cost) best = TileChoice{t, q};
   }
-  if (epi == EPI_DX) return c;
-  double best = c.split.s > 1 ? c.split.cost : tile_cost<T256>(rows_a, rows_b, nk, cus, 1.0, 1.0, 8.0);
-  const double t320 = allowed >> TILE_320 & 1 ? tile_cost<T320>(rows_a, rows_b, nk, cus, 1.25, 1.25, 8.0) : 1e300;
-  const double t192 = allowed >> TILE_192 & 1 ? tile_cost<T192>(rows_a, rows_b, nk, cus, 0.80, 0.80, 7.0) : 1e300;
-  const double t128 = allowed >> TILE_128 & 1 ? tile_cost<T128>(rows_a, rows_b, nk, cus, 0.60, 0.30, 4.0) : 1e300;
-  if (t320 < best) { best = t320; c.tile = TILE_320; }
-  if (t192 < best) { best = t192; c.tile = TILE_192; }
-  if (t128 < best) { best = t128; c.tile = TILE_128; }
-  if (c.tile != TILE_256) c.split = SplitPlan{0, 0, 1, 0.0};
-  if (c.tile == TILE_128 && can_split) c.split = split_plan128(tiles128, nk, cus);
-  return c;
+  return best;
 }
 
-// The tile shapes and split a launch may take: grouped forwards (row segments on 256- or 128-row boundaries)
-// no 192-row tiles and no split; segmented reductions no split (a piece would start inside a segment) and no
-// 256 x 320 tiles (that kernel variant spills registers).
+// The tile shapes a launch may take: grouped forwards (row segments on 256- or 128-row boundaries) no 192-row
+// tiles; segmented reductions no 256 x 320 tiles (that kernel variant spills registers).
 constexpr unsigned ALL_TILES = (1u << TILE_COUNT) - 1;
 unsigned allowed_tiles(bool grouped, bool ksegs) {
   unsigned m = ALL_TILES;
@@ -1395,16 +1517,17 @@ unsigned allowed_tiles(bool grouped, bool ksegs) {
   return m;
 }
 
-// Workspace for any schedule an entry may take: the larger of the T256 and T128 split plans' pieces (used when
-// the launch runs that tile shape, chosen or forced; other shapes leave it untouched).
-int64_t split_ws_bytes(int64_t rows_a, int64_t rows_b, int64_t kbytes) {
+// Workspace for any schedule an entry may take: the larger of the T256 and T128 plans' pieces (used when the launch
+// runs that tile shape, chosen or forced; other shapes leave it untouched).
+int64_t split_ws_bytes(bool bf16, int64_t rows_a, int64_t rows_b, int64_t kbytes) {
   const int cus = k2q_cu_count();
-  const int nk = (int)(kbytes / SBK);
-  const SplitPlan q = split_plan(((rows_a + 255) / 256) * ((rows_b + 255) / 256), nk, cus);
-  const SplitPlan q128 = split_plan128(((rows_a + 127) / 128) * ((rows_b + 127) / 128), nk, cus);
-  const int64_t b256 = q.s > 1 ? (int64_t)q.rem * q.s * 256 * 256 * 4 : 0;
-  const int64_t b128 = q128.s > 1 ? (int64_t)q128.rem * q128.s * 128 * 128 * 4 : 0;
-  return b256 > b128 ? b256 : b128;
+  int64_t bytes = 0;
+  for (int t : {TILE_256, TILE_128}) {
+    const SplitPlan q = tile_plan(t, bf16, rows_a, rows_b, (int)(kbytes / WBK), cus, true);
+    const int64_t b = q.s > 1 ? (int64_t)q.rem * q.s * TILE_COSTS[t].ta * TILE_COSTS[t].tb * 4 : 0;
+    bytes = b > bytes ? b : bytes;
+  }
+  return bytes;
 }
 
 template <int EPI, int MODE, class C, int NS>
@@ -1458,18 +1581,34 @@ int launch_full(const GemmArgs& p, hipStream_t st) {
 }
 
 // A split schedule: the pieces first (they fill the GPU for a short round), then the full tiles, then the fixup.
-// Split launches carry no segments (the caller runs grouped launches as full-K tiles).
+template <int EPI, class C, int MODE, int NS>
+int launch_split_as(const GemmArgs& p, const SplitPlan& q, hipStream_t st) {
+  // a segmented reduction's fixup reads no operands: its epilogue takes the base alone
+  constexpr int FNS = EPI == EPI_W8 ? NS : 0;
+  int rc;
+  if ((rc = set_lds<EPI, MODE, C, NS>())) return rc;
+  GemmArgsN<NS> ps;
+  GemmArgsN<FNS> pf;
+  if constexpr (NS > 0) ps = p;
+  else ps = slim(p);
+  if constexpr (FNS > 0) pf = p;
+  else pf = slim(p);
+  hipLaunchKernelGGL((gemm_nt_kernel<EPI, MODE, C, NS>), dim3((unsigned)(q.rem * q.s)), dim3(GT), C::LDS, st, ps);
+  if (q.dp_tiles > 0 && (rc = launch_full<EPI, C>(p, st))) return rc;
+  hipLaunchKernelGGL((gemm_fixup_kernel<EPI, C, FNS>), dim3((unsigned)(q.rem * fix_wgs_per_tile<C>())),
+                     dim3(64 * FIX_WAVES), 0, st, pf);
+  return K2Q_OK;
+}
+
 template <int EPI, class C>
 int launch_split(const GemmArgs& p, const SplitPlan& q, hipStream_t st) {
-  if (p.nseg > 0 || p.nks > 0) return K2Q_EINVAL;
-  int rc;
-  if ((rc = set_lds<EPI, MODE_PIECE, C, 0>()) || (rc = set_lds<EPI, MODE_FIXUP, C, 0>())) return rc;
-  const GemmArgsN<0> ps = slim(p);
-  hipLaunchKernelGGL((gemm_nt_kernel<EPI, MODE_PIECE, C, 0>), dim3((unsigned)(q.rem * q.s)), dim3(GT), C::LDS, st,
-                     ps);
-  if (q.dp_tiles > 0 && (rc = launch_full<EPI, C>(p, st))) return rc;
-  hipLaunchKernelGGL((gemm_nt_kernel<EPI, MODE_FIXUP, C, 0>), dim3((unsigned)q.rem), dim3(GT), C::LDS, st, ps);
-  return K2Q_OK;
+  if constexpr (EPI == EPI_W8) {
+    if (p.nseg > 0) return launch_split_as<EPI, C, MODE_PIECE, MAX_SEG>(p, q, st);
+  }
+  if constexpr (EPI == EPI_DXLIN) {
+    if (p.nks > 0) return launch_split_as<EPI, C, MODE_KPIECE, MAX_SEG>(p, q, st);
+  }
+  return launch_split_as<EPI, C, MODE_PIECE, 0>(p, q, st);
 }
 
 // B-tiles per group of the tile order.  A launch whose tiles all run at once (one round of full-K tiles, or a
@@ -1523,7 +1662,8 @@ int launch_gemm(GemmArgs p, void* ws, int64_t ws_bytes, hipStream_t st, int forc
   if (320 * ld_max >= 0x7fffffffLL) return K2Q_EUNSUPPORTED;
   if (forced >= TILE_COUNT || (EPI == EPI_DX && forced >= 0 && forced != TILE_256)) return K2Q_EINVAL;
   TileChoice c = choose_tile(EPI, p.rows_a, p.rows_b, p.kbytes, allowed_tiles(p.nseg > 0, p.nks > 0),
-                             p.nseg == 0 && p.nks == 0, forced, k2q_cu_count());
+                             ws != nullptr && (p.nks == 0 || p.kbytes / WBK >= KSEG_SPLIT_MIN), forced,
+                             k2q_cu_count());
   if (forced >= 0 && !(allowed_tiles(p.nseg > 0, p.nks > 0) >> forced & 1)) return K2Q_EINVAL;
   if (p.nseg > 0) {   // segments start on tile boundaries
     const int ta = c.tile == TILE_192 ? 192 : c.tile == TILE_128 ? 128 : 256;
@@ -1606,12 +1746,12 @@ int check_lora(const float* u, const float* lb, int64_t r) {
 
 extern "C" int64_t k2q_gemm_w8a8_ws_bytes(int64_t M, int64_t N, int64_t K) {
   if (check_common(M, N, K) || M <= K2Q_GEMV_MAX_M) return 0;
-  return split_ws_bytes(N, M, K);
+  return split_ws_bytes(false, N, M, K);
 }
 
 extern "C" int64_t k2q_gemm_dx_ws_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || K < K2Q_HADAMARD || K % K2Q_HADAMARD || N < 64 || N % 64) return 0;
-  return split_ws_bytes(K, M, 2 * N);
+  return split_ws_bytes(true, K, M, 2 * N);
 }
 
 extern "C" int k2q_gemm_w8a8(const int8_t* qx, const float* sx, const int8_t* qw, const float* sw,
@@ -1662,7 +1802,7 @@ extern "C" int k2q_gemm_w8a8_plan(int64_t M, int64_t N, int64_t K, int cus, int 
     if (split_pieces) *split_pieces = 1;
     return K2Q_TILE_GEMV;
   }
-  const TileChoice c = choose_tile(EPI_W8, N, M, K, allowed_tiles(grouped != 0, false), grouped == 0, TILE_AUTO, cus);
+  const TileChoice c = choose_tile(EPI_W8, N, M, K, allowed_tiles(grouped != 0, false), true, TILE_AUTO, cus);
   if (split_pieces) *split_pieces = c.tile == TILE_256 || c.tile == TILE_128 ? c.split.s : 1;
   return c.tile;
 }
@@ -1706,9 +1846,7 @@ extern "C" int k2q_gemm_w8a8_grouped(const int8_t* qx, const float* sx, int64_t 
   p.lora_rb = any_lora ? u : nullptr;
   p.r = any_lora ? (int)r : 0;
   p.ldr = (int)ldu;
-  (void)ws;
-  (void)ws_bytes;   // full-K tiles only: the split schedule's kernels take no segments
-  return launch_gemm<EPI_W8>(p, nullptr, 0, static_cast<hipStream_t>(stream));
+  return launch_gemm<EPI_W8>(p, ws, ws_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int k2q_gemm_w8a8_acc(const int8_t* qx, const int8_t* qw, int64_t M, int64_t N, int64_t K,
@@ -1744,7 +1882,7 @@ extern "C" int k2q_gemm_dx(const uint16_t* dy, const uint16_t* wt, int64_t M, in
 
 extern "C" int64_t k2q_gemm_bf16_ws_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || N % 4 || K < 64 || K % 64) return 0;
-  return split_ws_bytes(N, M, 2 * K);
+  return split_ws_bytes(true, N, M, 2 * K);
 }
 
 extern "C" int k2q_gemm_bf16(const uint16_t* x, const uint16_t* w, const float* bias, const float* u,
@@ -1784,6 +1922,12 @@ extern "C" int k2q_gemm_dx_lin(const uint16_t* dy, const uint16_t* wt, int64_t M
 
 extern "C" int k2q_gemm_dx_grouped(const k2q_dx_segment* seg, int64_t nseg, int64_t M, int64_t K, const float* g,
                                    int64_t ldg, const float* lora_a, int64_t r, uint16_t* dx, void* stream) {
+  return k2q_gemm_dx_grouped_ws(seg, nseg, M, K, g, ldg, lora_a, r, dx, nullptr, 0, stream);
+}
+
+extern "C" int k2q_gemm_dx_grouped_ws(const k2q_dx_segment* seg, int64_t nseg, int64_t M, int64_t K, const float* g,
+                                      int64_t ldg, const float* lora_a, int64_t r, uint16_t* dx, void* ws,
+                                      int64_t ws_bytes, void* stream) {
   if (!seg || nseg < 1 || nseg > MAX_SEG || M < 1 || K < 64 || K % 64 || !dx || !k2q_aligned(dx, 16))
     return K2Q_EINVAL;
   GemmArgs p{};
@@ -1806,7 +1950,7 @@ extern "C" int k2q_gemm_dx_grouped(const k2q_dx_segment* seg, int64_t nseg, int6
   p.rows_a = K; p.rows_b = M; p.kbytes = stages * WBK;
   p.out = dx; p.ldo = K;
   p.lora_rb = g; p.lora_ra = lora_a; p.r = g ? (int)r : 0; p.ldr = g ? (int)ldg : 0; p.lora_scale = 1.f;
-  return launch_gemm<EPI_DXLIN>(p, nullptr, 0, static_cast<hipStream_t>(stream));
+  return launch_gemm<EPI_DXLIN>(p, ws, ws_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int k2q_gemm_w4a8(const int8_t* qx, const float* sx, const uint8_t* qw4, const uint16_t* sw4,

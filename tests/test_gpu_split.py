@@ -1,0 +1,73 @@
+"""GPU tests of the split schedule over segments: a grouped W8A8 forward and a segmented input gradient whose last round
+of tiles is cut along the reduction, and the fixup launch that adds the pieces.
+
+W8A8 outputs equal the separate unsplit launches' bit for bit (int32 sums are exact, the epilogue is the same
+arithmetic).  The input gradient is checked on small whole numbers, whose sums every f32 order gives exactly
+(|sum| < 2^24), so the bf16 result must equal the float64 product rounded once.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,K,Ns,r", [(9, 6144, (512, 256), 16), (129, 16384, (256, 256, 512), 48),
+                                      (768, 6144, (16384, 16384), 16), (1300, 6144, (6144, 1536, 1536, 6144), 0),
+                                      (300, 6144, (1536, 1536, 1536), 16)])
+def test_grouped_split_equals_separate(k2, dev, M, K, Ns, r):
+    L = k2._lib
+    assert L.gemm_w8a8_plan(M, sum(Ns), K, grouped=True)[1] > 1          # the split schedule is taken
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    qx = torch.randint(-127, 128, (M, K), device=dev, dtype=torch.int8, generator=g)
+    sx = torch.rand(M, device=dev, generator=g) * 0.05 + 0.01
+    n = len(Ns)
+    u = torch.randn(M, n * r, device=dev, generator=g) if r else None
+    segs = []
+    for i, N in enumerate(Ns):
+        qw = torch.randint(-127, 128, (N, K), device=dev, dtype=torch.int8, generator=g)
+        sw = torch.rand(N, device=dev, generator=g) * 1e-3 + 1e-4
+        bias = torch.randn(N, device=dev, generator=g) if i % 2 else None
+        B = torch.randn(N, r, device=dev, generator=g) * 0.01 if r else None
+        segs.append((qw, sw, bias, B, i * r, 0.5 + i))
+    ys = L.gemm_w8a8_grouped(qx, sx, segs, u)
+    for y, (qw, sw, bias, B, col, sc) in zip(ys, segs):
+        ui = u[:, col:col + r].contiguous() if r else None
+        assert torch.equal(y, L.gemm_w8a8(qx, sx, qw, sw, bias, ui, B, sc, split=False))
+
+
+@pytest.mark.parametrize("M,K,Ns", [(9, 512, (3072, 64)), (130, 1024, (64, 3072, 192)), (768, 6144, (8192, 8192)),
+                                    (300, 6144, (1536, 6144, 1536, 6144)), (64, 640, (3136,))])
+def test_segmented_input_gradient_split_exact(k2, dev, M, K, Ns):
+    L = k2._lib
+    g = torch.Generator(device=dev).manual_seed(M + K + len(Ns))
+    dys = [torch.randint(-3, 4, (M, N), device=dev, generator=g).bfloat16() for N in Ns]
+    wts = [torch.randint(-3, 4, (K, N), device=dev, generator=g).bfloat16() for N in Ns]
+    A = torch.randint(-3, 4, (16, K), device=dev, generator=g).float()
+    gg = torch.randint(-3, 4, (M, 16), device=dev, generator=g).float()
+    ref = gg.double() @ A.double()
+    for d, w in zip(dys, wts):
+        ref += d.double() @ w.double().t()
+    dx = L.gemm_dx_grouped(list(zip(dys, wts)), gg, A)
+    assert torch.equal(dx, ref.bfloat16())
+    one = L.load().k2q_gemm_dx_ws_bytes(M, sum(Ns), K)
+    assert one > 0                                                        # the shape has a split schedule
+
+
+@pytest.mark.parametrize("M,N,K,r", [(130, 1028, 16384, 48), (33, 132, 12288, 16), (257, 260, 16384, 0),
+                                     (1000, 3072, 16384, 128)])
+def test_fixup_ragged_equals_unsplit(k2, dev, M, N, K, r):
+    """Widths that are not whole 16-byte rows, tiles partly past the matrix, and several LoRA chunks."""
+    L = k2._lib
+    assert L.gemm_w8a8_plan(M, N, K)[1] > 1
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    qx = torch.randint(-127, 128, (M, K), device=dev, dtype=torch.int8, generator=g)
+    qw = torch.randint(-127, 128, (N, K), device=dev, dtype=torch.int8, generator=g)
+    sx = torch.rand(M, device=dev, generator=g) * 0.05 + 0.01
+    sw = torch.rand(N, device=dev, generator=g) * 1e-3 + 1e-4
+    bias = torch.randn(N, device=dev, generator=g)
+    u = torch.randn(M, r, device=dev, generator=g) if r else None
+    B = torch.randn(N, r, device=dev, generator=g) * 0.01 if r else None
+    y = L.gemm_w8a8(qx, sx, qw, sw, bias, u, B, 0.5)
+    assert torch.equal(y, L.gemm_w8a8(qx, sx, qw, sw, bias, u, B, 0.5, split=False))
+    for t in ("256x256", "128x128"):
+        assert torch.equal(y, L.gemm_w8a8(qx, sx, qw, sw, bias, u, B, 0.5, tile=t)), t
