@@ -660,7 +660,7 @@ def linear_fwd(x2, qx, sx, codes_ready: bool, A, B, lora_scale: float, qw, sw, b
         nws = lib.k2q_linear_fwd_ws_bytes(wmode, M, N, K, r)
         # with u given, a call that takes u from the rotate/quant pass and whose GEMM does not split uses no ws
         unused = r and M > 8 and lib.k2q_linear_fwd_fuses_down(M, K, r) and \
-            (w4 or lib.k2q_gemm_w8a8_ws_bytes(M, N, K) == 0)
+            lib.k2q_linear_fwd_ws_bytes(wmode, M, N, K, 0) == 0
         plan = _FWD_WS.setdefault(key, (nws, 0 if unused else nws))
     nws = plan[1] if u is not None and not codes_ready else plan[0]
     ws = torch.empty((nws,), dtype=torch.uint8, device=dev) if nws > 0 else None

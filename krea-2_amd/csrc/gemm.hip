@@ -1184,9 +1184,9 @@ __global__ __launch_bounds__(64 * FIX_WAVES) void gemm_fixup_kernel(GemmArgsN<NS
 
 // ---------------------------------------------------------------------------------------------------------
 // W4A8: A operand = packed int4 weights (rows n, K/2 bytes per row), bf16 group scales sw4[g][n].
-// Tile 128 (n) x 128 (m) per 256-thread workgroup, three workgroups per CU (166 VGPRs) so that one wave's
-// per-group scaling runs while another's MFMAs do (wave priority follows the work left, see step()).
-// Wave w owns the 32 n-rows 32w..32w+31 and all 128 m, so every
+// Tile 128 (n) x 32 IB (m) per 256-thread workgroup, IB = 4, 2 or 1 (three, four or five workgroups per CU) so that
+// one wave's per-group scaling runs while another's MFMAs do (wave priority follows the work left, see step()).
+// Wave w owns the 32 n-rows 32w..32w+31 and all the tile's m, so every
 // packed weight byte is unpacked by exactly one wave.  The MFMA takes the x codes as its first operand, so
 // a lane's 16 results share one n (the lane's column) and need one group scale.  A stage is 128 of K,
 // double-buffered in LDS and filled by LDS-DMA from buffer resources (per-lane offsets fixed, the stage
@@ -1196,17 +1196,26 @@ __global__ __launch_bounds__(64 * FIX_WAVES) void gemm_fixup_kernel(GemmArgsN<NS
 // values 16*q in K order, so one v_mfma_i32_32x32x32_i8 per 32 of K sees 16x the true products (exact,
 // |16 acc_g| <= 16*64*127*8 < 2^20).  Each 64-wide group is accumulated in int32, converted once and
 // scaled: accf += float(acc_g) * s[g][n]; the 1/16 is folded into the final scale.  The per-group
-// convert + FMA (2 VALU ops per output per group) bounds this kernel, not the MFMAs.
+// convert + FMA (2 VALU ops per output per group) bounds this kernel on full grids, not the MFMAs.  Small grids
+// are bound by a workgroup's stage latency (0.6-1.2 us with a CU to itself) and, with few rows, by scaling rows past
+// M: they take lower tiles and cut the reduction into pieces whose f32 sums w4_fixup_kernel adds in order (w4_plan).
 constexpr int W4_BA = 128;                // n rows per tile
-constexpr int W4_BB = 128;                // m rows per tile
-constexpr int W4_IB = 4;                  // 32-row m blocks per wave (one 32-row n block)
 constexpr int W4_SA = W4_BA * 64;         // packed A bytes per stage (128 K codes per row)
-constexpr int W4_SB = W4_BB * WBK;        // B bytes per stage
 constexpr int W4_SS = 2 * W4_BA * 2;      // 2 groups x 128 n x bf16
-constexpr int W4_STAGE = W4_SA + W4_SB + W4_SS;
-constexpr int W4_G = 7;                   // DMA instructions per wave and stage: 2 A, 4 B, 1 scales
 constexpr int W4_CROW = 2 * W4_BA + 16;   // epilogue bf16 tile row (padded: rows m and m + 4 on other banks)
-static_assert(W4_BB * W4_CROW + 4 * W4_BB <= 2 * W4_STAGE, "epilogue tile and s_x fit the stage buffers");
+
+// Tile heights: IB blocks of 32 m rows per wave, and the workgroups per CU that their registers and LDS allow.
+template <int IB_>
+struct W4Tile {
+  static constexpr int IB = IB_, BB = 32 * IB;      // m rows per tile
+  static constexpr int SB = BB * WBK;               // B bytes per stage
+  static constexpr int STAGE = W4_SA + SB + W4_SS;
+  static constexpr int G = 3 + IB;                  // DMA instructions per wave and stage: 2 A, IB B, 1 scales
+  static constexpr int WPC = IB == 4 ? 3 : IB == 2 ? 4 : 5;
+  static constexpr int LDS = 2 * STAGE;
+  static_assert(BB * W4_CROW + 4 * BB <= LDS, "epilogue tile and s_x fit the stage buffers");
+  static_assert(WPC * LDS <= 160 * 1024, "gfx950 LDS is 160 KB per CU");
+};
 
 struct W4Args {
   const uint8_t* a;      // N x K/2 packed
@@ -1220,142 +1229,27 @@ struct W4Args {
   const float* lora_ra;
   int r;
   float lora_scale;
+  int s;                 // pieces per tile (1: none)
+  float* part;           // s > 1: the pieces' f32 sums, unit-major (16-byte unit 4 ib + q of thread t at 256 unit + t)
 };
 
 __device__ __forceinline__ int swz4(int row) { return (row >> 2) & 3; }
 
-template <int EPI>
-__global__ __launch_bounds__(256, 3) __attribute__((amdgpu_waves_per_eu(3, 3))) void gemm_w4_kernel(W4Args p) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][A | B | scales]
-
-  const uint32_t tiles_a = (uint32_t)((p.N + W4_BA - 1) / W4_BA);
-  const uint32_t tiles_b = (uint32_t)((p.M + W4_BB - 1) / W4_BB);
-  uint32_t ta, tb;
-  tile_coords(tiles_a, tiles_b, ta, tb);
-  const int64_t A0 = (int64_t)ta * W4_BA, B0 = (int64_t)tb * W4_BB;
-
-  const int t = threadIdx.x;
-  const int lane = t & 63;
+// Scales, bias, LoRA and the row-contiguous store of IB 32-row blocks starting at row B0 (columns A0 .. +127), the
+// workgroup's four waves owning 32 columns each: accf[ib][e] is n = A0 + 32 wave + c32, m = B0 + 32 ib + 8 (e / 4)
+// + 4 h + e % 4.  smem: 32 IB rows of W4_CROW bytes, then 32 IB floats.
+template <int EPI, int IB>
+__device__ __forceinline__ void w4_epilogue(const W4Args& p, v16f (&accf)[IB], int64_t A0, int64_t B0, uint8_t* smem) {
+  const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int h = lane >> 5, c32 = lane & 31;
-  const int64_t kb = p.K / 2;   // packed bytes per A row
-  const int64_t na = (p.N - A0) < W4_BA ? (p.N - A0) : W4_BA;
-  const int64_t nb = (p.M - B0) < W4_BB ? (p.M - B0) : W4_BB;
-
-  v16f accf[W4_IB];
-#pragma unroll
-  for (int j = 0; j < W4_IB; ++j) accf[j] = v16f{0.f};
-
-  // DMA sources, as offsets into buffer resources that start at the tile's first row (rows past the
-  // matrix end clamped onto its last row; never stored).  A: wave w fills rows 32w + 16i + l/4, physical
-  // chunk l%4; B: rows 32w + 8i + l/8, physical chunk l%8; scales: wave w copies group w/2, columns
-  // 64 (w&1) + 2l, 2l+1 with lanes 0-31.
-  const __amdgpu_buffer_rsrc_t ra = k2q_rsrc(p.a + A0 * kb, na * kb);
-  const __amdgpu_buffer_rsrc_t rb = k2q_rsrc(reinterpret_cast<const uint8_t*>(p.b) + B0 * p.K, nb * p.K);
-  const __amdgpu_buffer_rsrc_t rs = k2q_rsrc(p.s4, (p.K / 64) * p.N * 2);
-  int offa[2], offb[4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int lrow = 32 * wave + 16 * i + (lane >> 2);
-    const int rr = lrow < na ? lrow : (int)na - 1;
-    offa[i] = (int)(rr * kb) + 16 * ((lane & 3) ^ swz4(lrow));
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int lrow = 32 * wave + 8 * i + (lane >> 3);
-    const int rr = lrow < nb ? lrow : (int)nb - 1;
-    offb[i] = (int)(rr * p.K) + 16 * ((lane & 7) ^ swz(lrow));
-  }
-  int64_t ncol = A0 + 64 * (wave & 1) + 2 * (lane & 31);
-  ncol = ncol < p.N ? ncol : p.N - 2;
-  const int offs = (int)(((int64_t)(wave >> 1) * p.N + ncol) * 2);
-  auto issue = [&](int st, int slot) {
-    uint8_t* base = smem + slot * W4_STAGE;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, K2Q_LPTR(base + 1024 * (2 * wave + i)), 16, offa[i], st * 64, 0,
-                                               0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, K2Q_LPTR(base + W4_SA + 1024 * (4 * wave + i)), 16, offb[i],
-                                               st * WBK, 0, 0);
-    if (lane < 32)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rs, K2Q_LPTR(base + W4_SA + W4_SB + 256 * (wave >> 1) + 128 * (wave & 1)), 4, offs,
-          (int)(st * 4 * p.N), 0, 0);
-  };
-
-  auto compute = [&](int slot) {
-    const uint8_t* tA = smem + slot * W4_STAGE;
-    const uint8_t* tB = tA + W4_SA;
-    const uint16_t* tS = reinterpret_cast<const uint16_t*>(tB + W4_SB);
-    const int arow = 32 * wave + c32;
-#pragma unroll
-    for (int grp = 0; grp < 2; ++grp) {
-      v16i acc[W4_IB];
-#pragma unroll
-      for (int j = 0; j < W4_IB; ++j) acc[j] = v16i{0};
-#pragma unroll
-      for (int k2 = 0; k2 < 2; ++k2) {
-        const int kk = 2 * grp + k2;
-        const v2u w = *reinterpret_cast<const v2u*>(tA + arow * 64 + 16 * (kk ^ swz4(arow)) + 8 * h);
-        const v4i fa = v4i{(int)((w[0] << 4) & 0xF0F0F0F0u), (int)((w[1] << 4) & 0xF0F0F0F0u),
-                           (int)(w[0] & 0xF0F0F0F0u), (int)(w[1] & 0xF0F0F0F0u)};
-        v4i fb[W4_IB];
-#pragma unroll
-        for (int i = 0; i < W4_IB; ++i) fb[i] = frag(tB, 32 * i + c32, 2 * kk + h);
-#pragma unroll
-        for (int ib = 0; ib < W4_IB; ++ib)   // rows m (x codes), columns n (weights): lane c32 is one n
-          acc[ib] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[ib], fa, acc[ib], 0, 0, 0);
-      }
-      const float sv = bf16_bits_to_f32(tS[grp * W4_BA + arow]);
-#pragma unroll
-      for (int ib = 0; ib < W4_IB; ++ib)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) accf[ib][e] = __builtin_fmaf((float)acc[ib][e], sv, accf[ib][e]);
-      // One group's int32 accumulators live at a time: the scaled sums pass through here before the next
-      // group's fragment reads (the memory clobber keeps those below), so its MFMAs cannot be hoisted
-      // above this group's conversion.
-      asm volatile("" : "+v"(accf[0]), "+v"(accf[1]), "+v"(accf[2]), "+v"(accf[3])::"memory");
-    }
-  };
-
-  // Double-buffered: stage s+2 is fetched into stage s's slot once every wave is done with it.  Unrolled
-  // by two so that the slot, and with it every LDS address, is a compile-time offset.
-  const int ns = (int)(p.K / 128);
-  auto step = [&](int st, int slot) {
-    // Priority by work left (3 in the first quarter of the stages .. 0 in the last): under oldest-first
-    // issue the three workgroups sharing a CU otherwise drift apart, and the last one finishes alone with
-    // no other wave to fill its MFMA/VALU gaps.
-    const int lvl = (4 * (ns - st) - 1) / ns;   // 3 .. 0
-    if (lvl == 3) __builtin_amdgcn_s_setprio(3);
-    else if (lvl == 2) __builtin_amdgcn_s_setprio(2);
-    else if (lvl == 1) __builtin_amdgcn_s_setprio(1);
-    else __builtin_amdgcn_s_setprio(0);
-    compute(slot);
-    wait_vmcnt<0>();                                       // stage st+1
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of the slot have landed
-    lds_barrier();
-    if (st + 2 < ns) issue(st + 2, slot);
-  };
-  issue(0, 0);
-  issue(ns > 1 ? 1 : 0, 1);
-  wait_vmcnt<W4_G>();
-  lds_barrier();
-  for (int st = 0; st < ns; st += 2) {
-    step(st, 0);
-    if (st + 1 < ns) step(st + 1, 1);
-  }
-  wait_vmcnt<0>();   // no LDS-DMA may still be in flight when the workgroup's LDS is released
-
-  // accf[ib][e]: n = a0 + c32, m = B0 + 32 ib + 8 (e / 4) + 4 h + e % 4.
   const int64_t a0 = A0 + 32 * wave;
   if constexpr (EPI == EPI_ACC) {
     float* out = static_cast<float*>(p.out);
     const int64_t n = a0 + c32;
     if (n < p.N) {
 #pragma unroll
-      for (int ib = 0; ib < W4_IB; ++ib)
+      for (int ib = 0; ib < IB; ++ib)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int64_t m = B0 + 32 * ib + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -1364,17 +1258,18 @@ __global__ __launch_bounds__(256, 3) __attribute__((amdgpu_waves_per_eu(3, 3))) 
     }
   } else {
     // s_x (times 2^-7 for the rotations and 1/16 for the nibble placement) staged in LDS for the tile's
-    // 128 rows; scales, bias and LoRA applied in registers; then the bf16 tile goes through LDS (row m:
+    // rows; scales, bias and LoRA applied in registers; then the bf16 tile goes through LDS (row m:
     // 128 n, W4_CROW bytes) for row-contiguous stores.
+    constexpr int BB = 32 * IB;
     uint16_t* ctile = reinterpret_cast<uint16_t*>(smem);
-    float* sxs = reinterpret_cast<float*>(smem + W4_BB * W4_CROW);
+    float* sxs = reinterpret_cast<float*>(smem + BB * W4_CROW);
     lds_barrier();   // every wave is past its last fragment read
-    if (t < W4_BB) sxs[t] = p.sx[B0 + t < p.M ? B0 + t : p.M - 1] * (0.0078125f * 0.0625f);
+    if (t < BB) sxs[t] = p.sx[B0 + t < p.M ? B0 + t : p.M - 1] * (0.0078125f * 0.0625f);
     lds_barrier();
     const int64_t n = a0 + c32 < p.N ? a0 + c32 : p.N - 1;
     const float bi = p.bias ? p.bias[n] : 0.f;
 #pragma unroll
-    for (int ib = 0; ib < W4_IB; ++ib) {
+    for (int ib = 0; ib < IB; ++ib) {
       v16f f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1396,7 +1291,7 @@ __global__ __launch_bounds__(256, 3) __attribute__((amdgpu_waves_per_eu(3, 3))) 
     lds_barrier();
     const int cq = t & 31;                   // 4 n per thread, 8 rows per pass
     const int64_t n4 = A0 + 4 * cq;
-    const int rows = (int)nb;
+    const int rows = (int)(p.M - B0 < BB ? p.M - B0 : BB);
     if (n4 < p.N) {
       uint16_t* o = static_cast<uint16_t*>(p.out) + (B0 + (t >> 5)) * p.N + n4;
       const uint8_t* c = reinterpret_cast<const uint8_t*>(ctile) + (t >> 5) * W4_CROW + 8 * cq;
@@ -1410,17 +1305,260 @@ __global__ __launch_bounds__(256, 3) __attribute__((amdgpu_waves_per_eu(3, 3))) 
   }
 }
 
-template <int EPI>
-int launch_w4(const W4Args& p, hipStream_t st) {
-  constexpr int lds = 2 * W4_STAGE;
-  // Buffer-resource extents are 32-bit: a tile's rows of either operand and the whole scale array.
-  if (p.K * W4_BB >= (int64_t(1) << 31) || (p.K / 64) * p.N * 2 >= (int64_t(1) << 31)) return K2Q_EUNSUPPORTED;
-  static std::atomic<uint64_t> lds_set{0};
-  if (k2q_lds_limit_once(gemm_w4_kernel<EPI>, lds, lds_set)) return K2Q_ELAUNCH;
-  const int64_t tiles = ((p.N + W4_BA - 1) / W4_BA) * ((p.M + W4_BB - 1) / W4_BB);
+template <int EPI, class C, bool PIECE>
+__device__ __forceinline__ void w4_tile(const W4Args& p) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][A | B | scales]
+  constexpr int IB = C::IB;
+
+  const uint32_t tiles_a = (uint32_t)((p.N + W4_BA - 1) / W4_BA);
+  const uint32_t tiles_b = (uint32_t)((p.M + C::BB - 1) / C::BB);
+  uint32_t ta, tb;
+  tile_coords(tiles_a, tiles_b, ta, tb);
+  const int64_t A0 = (int64_t)ta * W4_BA, B0 = (int64_t)tb * C::BB;
+
+  const int t = threadIdx.x;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int h = lane >> 5, c32 = lane & 31;
+  const int64_t kb = p.K / 2;   // packed bytes per A row
+  const int64_t na = (p.N - A0) < W4_BA ? (p.N - A0) : W4_BA;
+  const int64_t nb = (p.M - B0) < C::BB ? (p.M - B0) : C::BB;
+
+  v16f accf[IB];
+#pragma unroll
+  for (int j = 0; j < IB; ++j) accf[j] = v16f{0.f};
+
+  // DMA sources, as offsets into buffer resources that start at the tile's first row (rows past the
+  // matrix end clamped onto its last row; never stored).  A: wave w fills rows 32w + 16i + l/4, physical
+  // chunk l%4; B: rows 8 IB w + 8i + l/8, physical chunk l%8; scales: wave w copies group w/2, columns
+  // 64 (w&1) + 2l, 2l+1 with lanes 0-31.
+  const __amdgpu_buffer_rsrc_t ra = k2q_rsrc(p.a + A0 * kb, na * kb);
+  const __amdgpu_buffer_rsrc_t rb = k2q_rsrc(reinterpret_cast<const uint8_t*>(p.b) + B0 * p.K, nb * p.K);
+  const __amdgpu_buffer_rsrc_t rs = k2q_rsrc(p.s4, (p.K / 64) * p.N * 2);
+  int offa[2], offb[IB];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int lrow = 32 * wave + 16 * i + (lane >> 2);
+    const int rr = lrow < na ? lrow : (int)na - 1;
+    offa[i] = (int)(rr * kb) + 16 * ((lane & 3) ^ swz4(lrow));
+  }
+#pragma unroll
+  for (int i = 0; i < IB; ++i) {
+    const int lrow = 8 * IB * wave + 8 * i + (lane >> 3);
+    const int rr = lrow < nb ? lrow : (int)nb - 1;
+    offb[i] = (int)(rr * p.K) + 16 * ((lane & 7) ^ swz(lrow));
+  }
+  int64_t ncol = A0 + 64 * (wave & 1) + 2 * (lane & 31);
+  ncol = ncol < p.N ? ncol : p.N - 2;
+  const int offs = (int)(((int64_t)(wave >> 1) * p.N + ncol) * 2);
+  auto issue = [&](int st, int slot) {
+    uint8_t* base = smem + slot * C::STAGE;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, K2Q_LPTR(base + 1024 * (2 * wave + i)), 16, offa[i], st * 64, 0,
+                                               0);
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, K2Q_LPTR(base + W4_SA + 1024 * (IB * wave + i)), 16, offb[i],
+                                               st * WBK, 0, 0);
+    if (lane < 32)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rs, K2Q_LPTR(base + W4_SA + C::SB + 256 * (wave >> 1) + 128 * (wave & 1)), 4, offs,
+          (int)(st * 4 * p.N), 0, 0);
+  };
+
+  auto compute = [&](int slot) {
+    const uint8_t* tA = smem + slot * C::STAGE;
+    const uint8_t* tB = tA + W4_SA;
+    const uint16_t* tS = reinterpret_cast<const uint16_t*>(tB + C::SB);
+    const int arow = 32 * wave + c32;
+#pragma unroll
+    for (int grp = 0; grp < 2; ++grp) {
+      v16i acc[IB];
+#pragma unroll
+      for (int j = 0; j < IB; ++j) acc[j] = v16i{0};
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        const int kk = 2 * grp + k2;
+        const v2u w = *reinterpret_cast<const v2u*>(tA + arow * 64 + 16 * (kk ^ swz4(arow)) + 8 * h);
+        const v4i fa = v4i{(int)((w[0] << 4) & 0xF0F0F0F0u), (int)((w[1] << 4) & 0xF0F0F0F0u),
+                           (int)(w[0] & 0xF0F0F0F0u), (int)(w[1] & 0xF0F0F0F0u)};
+        v4i fb[IB];
+#pragma unroll
+        for (int i = 0; i < IB; ++i) fb[i] = frag(tB, 32 * i + c32, 2 * kk + h);
+#pragma unroll
+        for (int ib = 0; ib < IB; ++ib)   // rows m (x codes), columns n (weights): lane c32 is one n
+          acc[ib] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[ib], fa, acc[ib], 0, 0, 0);
+      }
+      const float sv = bf16_bits_to_f32(tS[grp * W4_BA + arow]);
+#pragma unroll
+      for (int ib = 0; ib < IB; ++ib)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) accf[ib][e] = __builtin_fmaf((float)acc[ib][e], sv, accf[ib][e]);
+      // One group's int32 accumulators live at a time: the scaled sums pass through here before the next
+      // group's fragment reads (the memory clobber keeps those below), so its MFMAs cannot be hoisted
+      // above this group's conversion.
+#pragma unroll
+      for (int ib = 0; ib < IB; ++ib) asm volatile("" : "+v"(accf[ib]) : : "memory");
+    }
+  };
+
+  // Double-buffered: stage s+2 is fetched into stage s's slot once every wave is done with it.  Unrolled
+  // by two so that the slot, and with it every LDS address, is a compile-time offset.  A piece runs stages
+  // k0 .. k0 + ns - 1 of the reduction.
+  const int ns_all = (int)(p.K / 128);
+  int k0 = 0, ns = ns_all;
+  if constexpr (PIECE) {
+    k0 = (int)((int64_t)blockIdx.y * ns_all / p.s);
+    ns = (int)(((int64_t)blockIdx.y + 1) * ns_all / p.s) - k0;
+  }
+  auto step = [&](int st, int slot) {
+    // Priority by work left (3 in the first quarter of the stages .. 0 in the last): under oldest-first
+    // issue the workgroups sharing a CU otherwise drift apart, and the last one finishes alone with
+    // no other wave to fill its MFMA/VALU gaps.
+    const int lvl = (4 * (ns - st) - 1) / ns;   // 3 .. 0
+    if (lvl == 3) __builtin_amdgcn_s_setprio(3);
+    else if (lvl == 2) __builtin_amdgcn_s_setprio(2);
+    else if (lvl == 1) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+    compute(slot);
+    wait_vmcnt<0>();                                       // stage st+1
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of the slot have landed
+    lds_barrier();
+    if (st + 2 < ns) issue(k0 + st + 2, slot);
+  };
+  issue(k0, 0);
+  issue(k0 + (ns > 1 ? 1 : 0), 1);
+  wait_vmcnt<C::G>();
+  lds_barrier();
+  for (int st = 0; st < ns; st += 2) {
+    step(st, 0);
+    if (st + 1 < ns) step(st + 1, 1);
+  }
+  wait_vmcnt<0>();   // no LDS-DMA may still be in flight when the workgroup's LDS is released
+
+  if constexpr (PIECE) {   // park the sums for the fixup launch
+    float* dst = p.part + ((int64_t)blockIdx.y * tiles_a * tiles_b + (int64_t)ta * tiles_b + tb) * (W4_BA * C::BB);
+#pragma unroll
+    for (int ib = 0; ib < IB; ++ib)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<v4f*>(dst + ((4 * ib + q) * 256 + t) * 4) =
+            v4f{accf[ib][4 * q], accf[ib][4 * q + 1], accf[ib][4 * q + 2], accf[ib][4 * q + 3]};
+  } else {
+    w4_epilogue<EPI, IB>(p, accf, A0, B0, smem);
+  }
+}
+
+template <int EPI, class C, bool PIECE>
+__global__ __launch_bounds__(256, C::WPC) __attribute__((amdgpu_waves_per_eu(C::WPC, C::WPC)))
+void gemm_w4_kernel(W4Args p) { w4_tile<EPI, C, PIECE>(p); }
+
+// The pieces of 32 rows of a tile added in slice order (f32, a fixed order), then the tile kernel's epilogue:
+// workgroup (tile, ib).
+template <int EPI, class C>
+__global__ __launch_bounds__(256) void w4_fixup_kernel(W4Args p) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[32 * W4_CROW + 4 * 32];
+  const uint32_t tiles_b = (uint32_t)((p.M + C::BB - 1) / C::BB);
+  const int64_t tiles = (int64_t)((p.N + W4_BA - 1) / W4_BA) * tiles_b;
+  const int64_t A0 = (int64_t)(blockIdx.x / tiles_b) * W4_BA;
+  const int ib = (int)blockIdx.y;
+  const int64_t B0 = (int64_t)(blockIdx.x % tiles_b) * C::BB + 32 * ib;
+  if (B0 >= p.M) return;
+  v16f accf[1] = {v16f{0.f}};
+  const float* src = p.part + (int64_t)blockIdx.x * (W4_BA * C::BB) + (4 * ib * 256 + (int)threadIdx.x) * 4;
+  for (int sl = 0; sl < p.s; ++sl) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const v4f v = *reinterpret_cast<const v4f*>(src + q * 1024);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) accf[0][4 * q + i] += v[i];
+    }
+    src += tiles * (W4_BA * C::BB);
+  }
+  w4_epilogue<EPI, 1>(p, accf, A0, B0, smem);
+}
+
+// The schedule of a W4A8 launch: tile height (32 IB rows) and K-pieces per tile.
+struct W4Plan {
+  int ib, s;
+};
+
+int64_t w4_tiles(int64_t M, int64_t N, int ib) { return ((N + W4_BA - 1) / W4_BA) * ((M + 32 * ib - 1) / (32 * ib)); }
+
+int64_t w4_piece_bytes(int64_t M, int64_t N, const W4Plan& q) {
+  return q.s > 1 ? w4_tiles(M, N, q.ib) * q.s * W4_BA * 32 * q.ib * 4 : 0;
+}
+
+// The cheapest of the heights and 1-8 pieces, estimated in microseconds: a stage of a CU that runs w workgroups costs
+// a + b w (latency, then the scaling's VALU work), a round of CUs x workgroups-per-CU its stages + e, pieces 4.2 +
+// 0.262 per MB.  A partly filled round is priced between its fullest CUs and the average one.  Fitted to the measured
+// times of every height and split at 119 launches (M 1-8192, N 1024-18432, K 1024-16384): 1.5 % from the fastest
+// measured plan on average.  Against the 128-row tiles over the full reduction that every launch took before:
+// 1 x 3072 x 12288 108.5 -> 16.4 us, 333 x 3072 x 3072 30.3 -> 17.2, 768 x 6144 x 6144 69.6 -> 54.0, 1024 x 12288 ->
+// 3072 107.9 -> 65.9; from 2048 rows the 128-row tiles are the faster ones again (4096 x 3072 x 3072 55.1 against
+// 61.6 and 76.4 for 64 and 32 rows: the packed weights are unpacked and their scales read per tile row).
+W4Plan w4_plan(int64_t M, int64_t N, int64_t K, int cus, bool can_split) {
+  struct Cost {
+    int ib, wpc;
+    double a, b, e;
+  };
+  constexpr Cost kCosts[] = {{1, W4Tile<1>::WPC, 0.309, 0.152, 0.671},
+                             {2, W4Tile<2>::WPC, 0.450, 0.214, 0.364},
+                             {4, W4Tile<4>::WPC, 0.723, 0.340, 0.314}};
+  const int stages = (int)(K / 128);
+  W4Plan best{4, 1};
+  double best_us = 1e30;
+  for (const Cost& c : kCosts) {
+    const int64_t tiles = w4_tiles(M, N, c.ib), slots = (int64_t)cus * c.wpc;
+    for (int s = 1; s <= 8; ++s) {
+      if (s > 1 && (!can_split || tiles * s > slots || stages / s < 2)) break;
+      const int st = (stages + s - 1) / s;
+      const int64_t full = tiles * s / slots, rem = tiles * s - full * slots;
+      double us = 3.4 + (double)full * (st * (c.a + c.b * c.wpc) + c.e);
+      if (rem > 0) {
+        const double avg = (double)rem / cus, most = (double)((rem + cus - 1) / cus);
+        us += st * (c.a + c.b * (0.498 * most + 0.502 * (avg < 1.0 ? 1.0 : avg))) + c.e;
+      }
+      if (s > 1) us += 4.173 + 0.262 * (double)(tiles * s) * (W4_BA * 32 * c.ib * 4) * 1e-6;
+      if (us < best_us) {
+        best_us = us;
+        best = W4Plan{c.ib, s};
+      }
+    }
+  }
+  return best;
+}
+
+template <int EPI, class C>
+int launch_w4_tile(W4Args p, hipStream_t st) {
+  const int64_t tiles = w4_tiles(p.M, p.N, C::IB);
   if (tiles > 0x7fffffff) return K2Q_EUNSUPPORTED;
-  hipLaunchKernelGGL(gemm_w4_kernel<EPI>, dim3((unsigned)tiles), dim3(256), lds, st, p);
+  if (p.s > 1) {
+    static std::atomic<uint64_t> set_p{0};
+    if (k2q_lds_limit_once(gemm_w4_kernel<EPI, C, true>, C::LDS, set_p)) return K2Q_ELAUNCH;
+    hipLaunchKernelGGL((gemm_w4_kernel<EPI, C, true>), dim3((unsigned)tiles, (unsigned)p.s), dim3(256), C::LDS, st, p);
+    hipLaunchKernelGGL((w4_fixup_kernel<EPI, C>), dim3((unsigned)tiles, C::IB), dim3(256), 0, st, p);
+  } else {
+    static std::atomic<uint64_t> set_t{0};
+    if (k2q_lds_limit_once(gemm_w4_kernel<EPI, C, false>, C::LDS, set_t)) return K2Q_ELAUNCH;
+    hipLaunchKernelGGL((gemm_w4_kernel<EPI, C, false>), dim3((unsigned)tiles), dim3(256), C::LDS, st, p);
+  }
   return k2q_launch_status();
+}
+
+template <int EPI>
+int launch_w4(W4Args p, void* ws, int64_t ws_bytes, hipStream_t st) {
+  // Buffer-resource extents are 32-bit: a tile's rows of either operand and the whole scale array.
+  if (p.K * 128 >= (int64_t(1) << 31) || (p.K / 64) * p.N * 2 >= (int64_t(1) << 31)) return K2Q_EUNSUPPORTED;
+  W4Plan q = w4_plan(p.M, p.N, p.K, k2q_cu_count(), ws != nullptr);
+  if (q.s > 1 && (ws_bytes < w4_piece_bytes(p.M, p.N, q) || !k2q_aligned(ws, 16)))
+    q = w4_plan(p.M, p.N, p.K, k2q_cu_count(), false);   // no room for the pieces
+  p.s = q.s;
+  p.part = static_cast<float*>(ws);
+  if (q.ib == 1) return launch_w4_tile<EPI, W4Tile<1>>(p, st);
+  if (q.ib == 2) return launch_w4_tile<EPI, W4Tile<2>>(p, st);
+  return launch_w4_tile<EPI, W4Tile<4>>(p, st);
 }
 
 // Launch plans.  A launch's time is estimated per tile shape, in microseconds, and the cheapest plan taken:
@@ -1953,9 +2091,21 @@ extern "C" int k2q_gemm_dx_grouped_ws(const k2q_dx_segment* seg, int64_t nseg, i
   return launch_gemm<EPI_DXLIN>(p, ws, ws_bytes, static_cast<hipStream_t>(stream));
 }
 
+int64_t gemm_w4a8_ws_bytes(int64_t M, int64_t N, int64_t K) {
+  if (check_common(M, N, K)) return 0;
+  return w4_piece_bytes(M, N, w4_plan(M, N, K, k2q_cu_count(), true));
+}
+
 extern "C" int k2q_gemm_w4a8(const int8_t* qx, const float* sx, const uint8_t* qw4, const uint16_t* sw4,
                              const float* bias, const float* u, const float* lora_b, int64_t r,
                              float lora_scale, int64_t M, int64_t N, int64_t K, uint16_t* y, void* stream) {
+  return gemm_w4a8_impl(qx, sx, qw4, sw4, bias, u, lora_b, r, lora_scale, M, N, K, y, nullptr, 0,
+                        static_cast<hipStream_t>(stream));
+}
+
+int gemm_w4a8_impl(const int8_t* qx, const float* sx, const uint8_t* qw4, const uint16_t* sw4, const float* bias,
+                   const float* u, const float* lora_b, int64_t r, float lora_scale, int64_t M, int64_t N, int64_t K,
+                   uint16_t* y, void* ws, int64_t ws_bytes, hipStream_t st) {
   int rc = check_common(M, N, K);
   if (rc) return rc;
   if (!qx || !sx || !qw4 || !sw4 || !y) return K2Q_EINVAL;
@@ -1967,7 +2117,7 @@ extern "C" int k2q_gemm_w4a8(const int8_t* qx, const float* sx, const uint8_t* q
   p.a = qw4; p.s4 = sw4; p.b = qx; p.N = N; p.M = M; p.K = K;
   p.out = y; p.sx = sx; p.bias = bias;
   p.lora_rb = u; p.lora_ra = lora_b; p.r = u ? (int)r : 0; p.lora_scale = lora_scale;
-  return launch_w4<EPI_W8>(p, static_cast<hipStream_t>(stream));
+  return launch_w4<EPI_W8>(p, ws, ws_bytes, st);
 }
 
 extern "C" int k2q_gemm_w4a8_f32(const int8_t* qx, const uint8_t* qw4, const uint16_t* sw4, int64_t M,
@@ -1979,5 +2129,5 @@ extern "C" int k2q_gemm_w4a8_f32(const int8_t* qx, const uint8_t* qw4, const uin
     return K2Q_EINVAL;
   W4Args p{};
   p.a = qw4; p.s4 = sw4; p.b = qx; p.N = N; p.M = M; p.K = K; p.out = out;
-  return launch_w4<EPI_ACC>(p, static_cast<hipStream_t>(stream));
+  return launch_w4<EPI_ACC>(p, nullptr, 0, static_cast<hipStream_t>(stream));
 }

@@ -81,6 +81,12 @@ int gemm_w8a8_impl(const int8_t* qx, const float* sx, const int8_t* qw, const fl
                    int64_t M, int64_t N, int64_t K, uint16_t* y, void* ws, int64_t ws_bytes, int tile,
                    hipStream_t st);
 
+// k2q_gemm_w4a8 with a workspace for its K-pieces (gemm_w4a8_ws_bytes; null or too small: full-K tiles).
+int64_t gemm_w4a8_ws_bytes(int64_t M, int64_t N, int64_t K);
+int gemm_w4a8_impl(const int8_t* qx, const float* sx, const uint8_t* qw4, const uint16_t* sw4, const float* bias,
+                   const float* u, const float* lora_b, int64_t r, float lora_scale, int64_t M, int64_t N, int64_t K,
+                   uint16_t* y, void* ws, int64_t ws_bytes, hipStream_t st);
+
 // Status helpers for the C ABI.
 static inline int k2q_launch_status() {
   hipError_t e = hipGetLastError();

@@ -142,7 +142,7 @@ FwdLayout fwd_layout(int wmode, int64_t M, int64_t N, int64_t K, int64_t r) {
     off += align256(a > b ? a : b);
   }
   L.gemm_off = off;
-  if (wmode == K2Q_WMODE_W8) off += align256(k2q_gemm_w8a8_ws_bytes(M, N, K));
+  off += align256(wmode == K2Q_WMODE_W8 ? k2q_gemm_w8a8_ws_bytes(M, N, K) : gemm_w4a8_ws_bytes(M, N, K));
   L.total = off;
   return L;
 }
@@ -242,6 +242,6 @@ extern "C" int k2q_linear_fwd(const uint16_t* x, int64_t ldx, int64_t M, int64_t
   if (wmode == K2Q_WMODE_W8)
     return gemm_w8a8_impl(qx, sx, static_cast<const int8_t*>(qw), static_cast<const float*>(sw), bias, uu, parts,
                           M * rr, lora_a ? lora_b : nullptr, rr, lora_scale, M, N, K, y, gws, gws_bytes, -1, st);
-  return k2q_gemm_w4a8(qx, sx, static_cast<const uint8_t*>(qw), static_cast<const uint16_t*>(sw), bias, uu,
-                       lora_a ? lora_b : nullptr, rr, lora_scale, M, N, K, y, stream);
+  return gemm_w4a8_impl(qx, sx, static_cast<const uint8_t*>(qw), static_cast<const uint16_t*>(sw), bias, uu,
+                        lora_a ? lora_b : nullptr, rr, lora_scale, M, N, K, y, gws, gws_bytes, st);
 }
