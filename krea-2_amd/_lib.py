@@ -5,10 +5,14 @@ Every wrapper validates shapes, dtypes, devices and contiguity on the host and r
 run on ``torch.cuda.current_stream()`` of the tensors' device.  Outputs are allocated with ``torch.empty``
 (PyTorch's caching allocator owns all memory).  There is no fallback: if the library or a gfx950 GPU is
 missing, the call raises.
+
+The wrappers that a linear's forward and backward call go through ``_k2q_native`` (``csrc/binding.cpp``): it checks
+the same arguments, allocates and calls the library; what it refuses comes back here for the error's text.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import threading
 from pathlib import Path
 
@@ -97,7 +101,10 @@ _SIGNATURES = {
 }
 EXPORTS = tuple(_SIGNATURES)
 
+NATIVE_PATH = Path(__file__).resolve().parent / "_k2q_native.so"
+
 _lib = None
+_native = None          # the binding module, its entry points bound to _lib's
 _lock = threading.Lock()
 _device_ok: dict[int, bool] = {}
 
@@ -116,8 +123,41 @@ def load() -> ctypes.CDLL:
                 fn = getattr(lib, name)
                 fn.argtypes = args
                 fn.restype = res
+            _bind_native(lib)
             _lib = lib
     return _lib
+
+
+def _bind_native(lib) -> None:
+    global _native
+    if not NATIVE_PATH.exists():
+        raise RuntimeError(f"{NATIVE_PATH} is not built; run krea-2_amd/build.py")
+    spec = importlib.util.spec_from_file_location("_k2q_native", NATIVE_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _SIGNATURES}, _stream_of_index)
+    _native = mod
+
+
+def _fast():
+    """The binding module (the library loaded)."""
+    if _native is None:
+        load()
+    return _native
+
+
+def _refused(rc, name: str, call, *checks):
+    """What a native wrapper that returned no tensors (``rc``) comes to: the library's status as an error, or the
+    arguments' checks (each raises what it finds; the last marks the device as gfx950) and the call once more."""
+    if rc is None:
+        for check in checks:
+            check()
+        rc = call()
+        if rc is None:
+            raise ValueError(f"{name}: the arguments do not match what the kernels take")
+    if rc.__class__ is int:
+        _check(rc, name)
+    return rc
 
 
 def version() -> str:
@@ -144,6 +184,9 @@ def _stream(dev: torch.device) -> int:
     return torch.cuda.current_stream(dev).cuda_stream
 
 
+_stream_of_index = _raw_stream or (lambda i: torch.cuda.current_stream(i).cuda_stream)
+
+
 def _device_check(dev: torch.device) -> None:
     if dev.type != "cuda":
         raise RuntimeError(f"k2q kernels need a gfx950 GPU tensor, got device {dev}")
@@ -151,6 +194,8 @@ def _device_check(dev: torch.device) -> None:
     if idx not in _device_ok:
         with torch.cuda.device(idx):
             _device_ok[idx] = load().k2q_check_device() == K2Q_OK
+        if _device_ok[idx]:
+            _native.device_checked(idx)
     if not _device_ok[idx]:
         raise RuntimeError(f"device cuda:{idx} is not gfx950 (MI355X); the k2q kernels are built for gfx950 only")
 
@@ -386,27 +431,34 @@ def quant_weight_i4(w: torch.Tensor):
 # ----------------------------------------------------------------------------------------------------------
 def lora_down(x: torch.Tensor, A: torch.Tensor) -> torch.Tensor:
     """``u = x.f32 @ A^T`` (M, r) f32; ``x`` (M,K) bf16, ``A`` (r,K) f32."""
+    u = _fast().lora_down(x, A)
+    if u.__class__ is torch.Tensor:
+        return u
+    return _refused(u, "k2q_lora_down", lambda: _native.lora_down(x, A), lambda: _check_lora_down(x, A))
+
+
+def _check_lora_down(x, A) -> None:
     _need(x, "x", torch.bfloat16, 2)
     dev = x.device
     _need(A, "lora_A", torch.float32, 2, dev)
-    M, K = x.shape
-    r = A.shape[0]
-    if A.shape[1] != K:
-        raise ValueError(f"lora_A has in_features {A.shape[1]}, x has {K}")
-    _check_rank(r)
+    if A.shape[1] != x.shape[1]:
+        raise ValueError(f"lora_A has in_features {A.shape[1]}, x has {x.shape[1]}")
+    _check_rank(A.shape[0])
     _device_check(dev)
-    lib = load()
-    nws = lib.k2q_lora_down_ws_bytes(M, K, r)
-    ws = torch.empty((nws // 4,), dtype=torch.float32, device=dev) if nws else None
-    u = torch.empty((M, r), dtype=torch.float32, device=dev)
-    _check(lib.k2q_lora_down(_ptr(x), M, K, K, _ptr(A), r, _ptr(ws), nws, _ptr(u), _stream(dev)), "k2q_lora_down")
-    return u
 
 
 def lora_grads(dy, x, u, lora_b, lora_scale: float):
     """LoRA gradients (the autograd of ``lora.py:47-48``): ``g = s dy B`` (M,r), ``dA = g^T x`` (r,K) when
     ``x`` is given, ``dB = s dy^T u`` (N,r) when ``u`` is given; all f32.  ``dy`` (M,N) and ``x`` (M,K) bf16,
     ``u`` (M,r) and ``lora_b`` (N,r) f32.  Returns ``(g, dA | None, dB | None)``."""
+    r = _fast().lora_grads(dy, x, u, lora_b, lora_scale)
+    if r.__class__ is tuple:
+        return r
+    return _refused(r, "k2q_lora_grads", lambda: _native.lora_grads(dy, x, u, lora_b, lora_scale),
+                    lambda: _check_lora_grads(dy, x, u, lora_b))
+
+
+def _check_lora_grads(dy, x, u, lora_b) -> None:
     _need(dy, "dy", torch.bfloat16, 2)
     dev = dy.device
     M, N = dy.shape
@@ -417,27 +469,16 @@ def lora_grads(dy, x, u, lora_b, lora_scale: float):
     _check_rank(r)
     if N % HADAMARD_BLOCK:
         raise ValueError(f"out_features={N} must be a multiple of {HADAMARD_BLOCK} for the LoRA gradients")
-    K = HADAMARD_BLOCK
     if x is not None:
         _need(x, "x", torch.bfloat16, 2, dev)
         if x.shape[0] != M:
             raise ValueError("x rows != dy rows")
-        K = x.shape[1]
-        _check_k(K)
+        _check_k(x.shape[1])
     if u is not None:
         _need(u, "u", torch.float32, 2, dev)
         if u.shape != (M, r):
             raise ValueError(f"u must be {(M, r)}, got {tuple(u.shape)}")
     _device_check(dev)
-    lib = load()
-    nws = lib.k2q_lora_grads_ws_bytes(M, N, K, r)
-    ws = torch.empty((nws,), dtype=torch.uint8, device=dev)
-    g = torch.empty((M, r), dtype=torch.float32, device=dev)
-    dA = torch.empty((r, K), dtype=torch.float32, device=dev) if x is not None else None
-    dB = torch.empty((N, r), dtype=torch.float32, device=dev) if u is not None else None
-    _check(lib.k2q_lora_grads(_ptr(dy), _ptr(x), _ptr(u), _ptr(lora_b), r, float(lora_scale), M, N, K, _ptr(g),
-                              _ptr(dA), _ptr(dB), _ptr(ws), nws, _stream(dev)), "k2q_lora_grads")
-    return g, dA, dB
 
 
 LORA_GROUP_MAX = 8     # members per k2q_lora_grads_grouped call
@@ -616,11 +657,6 @@ def gemm_w8a8(qx, sx, qw, sw, bias=None, u=None, lora_b=None, lora_scale: float 
 WMODE_W8, WMODE_W4 = 0, 1
 
 
-# workspace bytes of k2q_linear_fwd per (wmode, M, N, K, r), as (any call, a call with u given and codes not
-# given): pure functions of the shape and the device's CU count (one GPU model per process here), asked once per shape
-_FWD_WS: dict = {}
-
-
 def linear_fwd_fuses_down(M: int, K: int, r: int) -> bool:
     """Whether :func:`linear_fwd` (codes not given, rank ``r`` factors) takes u from the rotate/quant pass."""
     return bool(load().k2q_linear_fwd_fuses_down(M, K, r))
@@ -635,12 +671,20 @@ def linear_fwd(x2, qx, sx, codes_ready: bool, A, B, lora_scale: float, qw, sw, b
     ``(y, None)``.  The module's per-call entry: the weights and factors come from the module (their shapes
     fixed when it was built), so only the relations a foreign call needs are checked here, cheaply; the library
     checks pointers and alignment again.  ``x2`` (M,K) bf16 rows of stride ``x2.stride(0)``."""
+    r = _fast().linear_fwd(x2, qx, sx, codes_ready, A, B, lora_scale, qw, sw, bias, w4, need_u)
+    if r.__class__ is tuple:
+        return r
+    return _refused(r, "k2q_linear_fwd", lambda: _native.linear_fwd(x2, qx, sx, codes_ready, A, B, lora_scale, qw, sw,
+                                                                    bias, w4, need_u),
+                    lambda: _check_linear_fwd(x2, qx, sx, A, B, qw, bias))
+
+
+def _check_linear_fwd(x2, qx, sx, A, B, qw, bias) -> None:
     M, K = x2.shape
     N = qw.shape[0]
     dev = x2.device
     if x2.dtype != torch.bfloat16 or x2.stride(1) != 1 or qw.device != dev or qx.shape != (M, K) or sx.shape != (M,):
         raise ValueError("linear_fwd: x / code buffers do not match the layer")
-    r = 0
     if A is not None:
         r = A.shape[0]
         if A.shape != (r, K) or B.shape != (N, r) or A.dtype != torch.float32 or B.dtype != torch.float32 \
@@ -650,24 +694,11 @@ def linear_fwd(x2, qx, sx, codes_ready: bool, A, B, lora_scale: float, qw, sw, b
     if bias is not None and (bias.shape != (N,) or bias.dtype != torch.float32 or bias.device != dev):
         raise ValueError("linear_fwd: bias does not match the layer")
     _device_check(dev)
-    lib = load()
-    wmode = WMODE_W4 if w4 else WMODE_W8
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-    u = torch.empty((M, r), dtype=torch.float32, device=dev) if r and (need_u or M <= 8) else None
-    key = (wmode, M, N, K, r)
-    plan = _FWD_WS.get(key)
-    if plan is None:
-        nws = lib.k2q_linear_fwd_ws_bytes(wmode, M, N, K, r)
-        # with u given, a call that takes u from the rotate/quant pass and whose GEMM does not split uses no ws
-        unused = r and M > 8 and lib.k2q_linear_fwd_fuses_down(M, K, r) and \
-            lib.k2q_linear_fwd_ws_bytes(wmode, M, N, K, 0) == 0
-        plan = _FWD_WS.setdefault(key, (nws, 0 if unused else nws))
-    nws = plan[1] if u is not None and not codes_ready else plan[0]
-    ws = torch.empty((nws,), dtype=torch.uint8, device=dev) if nws > 0 else None
-    _check(lib.k2q_linear_fwd(x2.data_ptr(), x2.stride(0), M, K, qx.data_ptr(), sx.data_ptr(), int(codes_ready),
-                              _ptr(A), _ptr(B), r, float(lora_scale), _ptr(u), wmode, qw.data_ptr(), sw.data_ptr(),
-                              _ptr(bias), N, y.data_ptr(), _ptr(ws), nws, _stream(dev)), "k2q_linear_fwd")
-    return y, (u if need_u else None)
+
+
+def alloc_codes(x2):
+    """The ``(int8 (M,K), f32 (M,))`` buffers that :func:`linear_fwd` fills with ``x2``'s codes and scales."""
+    return _fast().alloc_codes(x2)
 
 
 def gemm_w8a8_grouped(qx, sx, segments, u=None):
@@ -789,6 +820,13 @@ def gemm_w4a8_f32(qx, q4, s4) -> torch.Tensor:
 def dx_weight(qw, sw, *, w4: bool = False) -> torch.Tensor:
     """The effective weight of the straight-through forward, ``bf16(2^-7 W_hat R)^T`` (K,N): what
     :func:`gemm_dx` builds on every call unless it is handed one (``wt=``)."""
+    wt = _fast().dx_weight(qw, sw, w4)
+    if wt.__class__ is torch.Tensor:
+        return wt
+    return _refused(wt, "k2q_dx_prep_eff", lambda: _native.dx_weight(qw, sw, w4), lambda: _check_dx_weight(qw, sw, w4))
+
+
+def _check_dx_weight(qw, sw, w4: bool) -> None:
     dev = qw.device
     if w4:
         _need(qw, "q_w4", torch.uint8, 2, dev)
@@ -806,10 +844,6 @@ def dx_weight(qw, sw, *, w4: bool = False) -> torch.Tensor:
     if N % 64:
         raise ValueError(f"out_features={N} must be a multiple of 64 for the input-gradient GEMM")
     _device_check(dev)
-    wt = torch.empty((K, N), dtype=torch.bfloat16, device=dev)
-    _check(load().k2q_dx_prep_eff(None if w4 else _ptr(qw), None if w4 else _ptr(sw), _ptr(qw) if w4 else None,
-                                  _ptr(sw) if w4 else None, N, K, _ptr(wt), _stream(dev)), "k2q_dx_prep_eff")
-    return wt
 
 
 def gemm_dx(dy, qw, sw, *, w4: bool = False, g=None, lora_a=None, split: bool = True,
@@ -818,6 +852,12 @@ def gemm_dx(dy, qw, sw, *, w4: bool = False, g=None, lora_a=None, split: bool = 
     scaled (``lora_scale * dy @ lora_B``), ``lora_a`` (r,K) f32.  ``fold_rotation`` (default) builds the
     effective weight ``bf16(2^-7 W_hat R)^T`` (or takes it as ``wt``, from :func:`dx_weight`) and runs the
     plain GEMM; otherwise ``bf16(W_hat)^T`` and the GEMM with the inverse rotation in its epilogue."""
+    if wt is not None and fold_rotation and split:
+        dx = _fast().gemm_dx(dy, wt, g, lora_a, qw, sw, w4)
+        if dx.__class__ is torch.Tensor:
+            return dx
+        if dx.__class__ is int:
+            _check(dx, "k2q_gemm_dx")
     _need(dy, "dy", torch.bfloat16, 2)
     dev = dy.device
     M, N = dy.shape
@@ -945,18 +985,28 @@ def _fp8_operands(q, s):
 
 def dequant_fp8(q, s, transpose: bool = False) -> torch.Tensor:
     """``bf16(q * s)`` per element (``quantize.py:49``): (N,K), or (K,N) with ``transpose``."""
-    N, K = _fp8_operands(q, s)
+    w = _fast().dequant_fp8(q, s, transpose)
+    if w.__class__ is torch.Tensor:
+        return w
+    return _refused(w, "k2q_dequant_fp8", lambda: _native.dequant_fp8(q, s, transpose),
+                    lambda: _check_dequant_fp8(q, s, transpose))
+
+
+def _check_dequant_fp8(q, s, transpose: bool) -> None:
+    N, _ = _fp8_operands(q, s)
     if transpose and N % 8:
         raise ValueError("the transposed dequantization needs out_features % 8 == 0")
     _device_check(q.device)
-    out = torch.empty((K, N) if transpose else (N, K), dtype=torch.bfloat16, device=q.device)
-    _check(load().k2q_dequant_fp8(_ptr(q), _ptr(s), N, K, int(transpose), _ptr(out), _stream(q.device)),
-           "k2q_dequant_fp8")
-    return out
 
 
 def gemm_bf16(x, w, bias=None, u=None, lora_b=None, lora_scale: float = 1.0, *, split: bool = True) -> torch.Tensor:
     """``y = bf16(x w^T + bias) + LoRA`` (``quantize.py:51`` + ``lora.py:47-48``); x (M,K), w (N,K) bf16."""
+    if split:
+        y = _fast().gemm_bf16(x, w, bias, u, lora_b, lora_scale)
+        if y.__class__ is torch.Tensor:
+            return y
+        if y.__class__ is int:
+            _check(y, "k2q_gemm_bf16")
     _need(x, "x", torch.bfloat16, 2)
     dev = x.device
     _need(w, "w", torch.bfloat16, 2, dev)
@@ -1005,6 +1055,12 @@ def gemm_dx_fp8(dy, q, s, *, g=None, lora_a=None, split: bool = True) -> torch.T
     lib = load()
     st = _stream(dev)
     wt = dequant_fp8(q, s, transpose=True)
+    if split:
+        dx = _native.gemm_dx(dy, wt, g, lora_a, None, None, False)
+        if dx.__class__ is torch.Tensor:
+            return dx
+        if dx.__class__ is int:
+            _check(dx, "k2q_gemm_dx_lin")
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
     ws, nws = _workspace(lib.k2q_gemm_dx_ws_bytes(M, N, K) if split else 0, dev)
     _check(lib.k2q_gemm_dx_lin(_ptr(dy), _ptr(wt), M, N, K, _ptr(g), _ptr(lora_a) if r else None, r, _ptr(dx),

@@ -86,7 +86,7 @@ class LoRALinear(nn.Module):
         A, B = self.lora_A, self.lora_B
         if A.dtype != torch.float32:
             A, B = A.float(), B.float()
-        extra = _padded_rank(self.rank) - self.rank
+        extra = -self.rank % _lib.RANK_ALIGN
         if extra:
             A = F.pad(A, (0, 0, 0, extra))
             B = F.pad(B, (0, extra))
@@ -94,12 +94,13 @@ class LoRALinear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         s = self.scale * self.scale_mul
-        if isinstance(self.base, _HIP_BASES):
+        base = self.base
+        if isinstance(base, _HIP_BASES):
             if s == 0.0:
-                return self.base(x)
+                return base(x)
             A, B = self._kernel_factors()
-            return self.base.forward_lora(x, A, B, s)
-        y = self.base(x)
+            return base.forward_lora(x, A, B, s)
+        y = base(x)
         if s == 0.0:
             return y
         return y + s * ((x.to(self.lora_A.dtype) @ self.lora_A.t()) @ self.lora_B.t()).to(y.dtype)

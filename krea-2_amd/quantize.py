@@ -45,7 +45,8 @@ class _SharedInputQuant:
 
     @staticmethod
     def _key(x: torch.Tensor):
-        return (x._version, x.data_ptr(), tuple(x.shape), tuple(x.stride()), x.device, _lib._stream(x.device))
+        dev = x.device
+        return (x._version, x.data_ptr(), x.shape, x.stride(), dev, _lib._stream(dev))
 
     def lookup(self, x: torch.Tensor, x2: torch.Tensor):
         key = self._key(x)
@@ -82,6 +83,12 @@ class _SharedInputQuant:
 
 
 shared_input_quant = _SharedInputQuant()
+
+
+def _token_rows(x: torch.Tensor, K: int) -> torch.Tensor:
+    """``x`` as (tokens, K) rows the kernels take: contiguous and 16-byte aligned (``x`` itself when it is that)."""
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
+    return x2 if x2.is_contiguous() and x2.data_ptr() % 16 == 0 else x2.contiguous()
 
 
 def _check_out_features(N: int) -> None:
@@ -244,9 +251,9 @@ class ConvRotLinear(nn.Module):
                f"bias={self.bias is not None}"
 
     def _bias_f32(self):
-        if self.bias is None:
-            return None
         b = self.bias
+        if b is None:
+            return None
         return b if b.dtype == torch.float32 and b.is_contiguous() else b.float().contiguous()
 
     def forward_lora(self, x: torch.Tensor, lora_A: torch.Tensor | None, lora_B: torch.Tensor | None,
@@ -256,20 +263,12 @@ class ConvRotLinear(nn.Module):
             raise ValueError(f"x has {x.shape[-1]} features, layer expects {self.in_features}")
         if x.dtype != torch.bfloat16:
             raise NotImplementedError(f"ConvRotLinear runs bf16 activations (the DiT dtype); got {x.dtype}")
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, self.in_features)
-        if not x2.is_contiguous() or x2.data_ptr() % 16:
-            x2 = x2.contiguous()
-        M = x2.shape[0]
-        if M == 0:
-            return x.new_empty(*lead, self.out_features)
+        x2 = _token_rows(x, self.in_features)
+        if x2.shape[0] == 0:
+            return x.new_empty(*x.shape[:-1], self.out_features)
         key, codes = shared_input_quant.find(x)
         ready = codes is not None
-        if ready:
-            qx, sx = codes
-        else:
-            qx = torch.empty((M, self.in_features), dtype=torch.int8, device=x2.device)
-            sx = torch.empty((M,), dtype=torch.float32, device=x2.device)
+        qx, sx = codes if ready else _lib.alloc_codes(x2)
         w4 = self.mode == "w4a8"
         grad = torch.is_grad_enabled() and (x2.requires_grad or (lora_A is not None and
                                                                   (lora_A.requires_grad or lora_B.requires_grad)))
@@ -281,7 +280,7 @@ class ConvRotLinear(nn.Module):
                                    self.weight_scale, self._bias_f32(), w4, need_u=False)
         if not ready:
             shared_input_quant.keep(x, key, qx, sx)
-        return y.reshape(*lead, self.out_features)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_features)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.forward_lora(x, None, None, 0.0)
@@ -343,15 +342,20 @@ def set_dx_weight_cache(model: nn.Module, enable: bool = True) -> int:
 # ----------------------------------------------------------------------------------------------------------
 # fp8-e4m3 weight-only base: the reference's own quantized Linear (quantize.py:23-51), on the same kernels
 # ----------------------------------------------------------------------------------------------------------
+def _fp8_forward(x2, lora_A, lora_B, q, scale, bias, lora_scale):
+    """``(y, u | None)``: the weight dequantized to bf16, the down-projection, the bf16 GEMM."""
+    w = _lib.dequant_fp8(q, scale)            # the reference's per-forward bf16 temporary
+    u = _lib.lora_down(x2, lora_A) if lora_A is not None else None
+    return _lib.gemm_bf16(x2, w, bias, u, lora_B, lora_scale), u
+
+
 class _Fp8LinearFn(torch.autograd.Function):
     """Forward ``quantize.py:48-51`` (dequantize to bf16, bf16 GEMM with f32 accumulation, bias) with the LoRA
     term of ``lora.py:47-48`` fused; backward ``dX = dY W_deq + g A``, ``dA = g^T x``, ``dB = s dY^T u``."""
 
     @staticmethod
     def forward(ctx, x2, lora_A, lora_B, q, scale, bias, lora_scale):
-        w = _lib.dequant_fp8(q, scale)            # the reference's per-forward bf16 temporary
-        u = _lib.lora_down(x2, lora_A) if lora_A is not None else None
-        y = _lib.gemm_bf16(x2, w, bias, u, lora_B, lora_scale)
+        y, u = _fp8_forward(x2, lora_A, lora_B, q, scale, bias, lora_scale)
         ctx.lora_scale = lora_scale
         ctx.save_for_backward(x2 if lora_A is not None else None, u, lora_A, lora_B, q, scale)
         return y
@@ -436,17 +440,18 @@ class Fp8Linear(nn.Module):
             raise ValueError(f"x has {x.shape[-1]} features, layer expects {self.in_features}")
         if x.dtype != torch.bfloat16:
             raise NotImplementedError(f"Fp8Linear runs bf16 activations (the DiT dtype); got {x.dtype}")
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, self.in_features)
-        if not x2.is_contiguous() or x2.data_ptr() % 16:
-            x2 = x2.contiguous()
+        x2 = _token_rows(x, self.in_features)
         if x2.shape[0] == 0:
-            return x.new_empty(*lead, self.out_features)
+            return x.new_empty(*x.shape[:-1], self.out_features)
         # the reference adds the bias in x.dtype (quantize.py:50): round it to bf16 first
         b = self.bias.to(torch.bfloat16).float().contiguous() if self.bias is not None else None
         scale = self.scale.to(torch.bfloat16).contiguous()
-        y = _Fp8LinearFn.apply(x2, lora_A, lora_B, self.weight_fp8, scale, b, float(lora_scale))
-        return y.reshape(*lead, self.out_features)
+        if torch.is_grad_enabled() and (x2.requires_grad or (lora_A is not None and
+                                                             (lora_A.requires_grad or lora_B.requires_grad))):
+            y = _Fp8LinearFn.apply(x2, lora_A, lora_B, self.weight_fp8, scale, b, float(lora_scale))
+        else:   # nothing to differentiate: no autograd node
+            y, _ = _fp8_forward(x2, lora_A, lora_B, self.weight_fp8, scale, b, float(lora_scale))
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_features)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.forward_lora(x, None, None, 0.0)
