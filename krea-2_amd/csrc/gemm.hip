@@ -129,10 +129,9 @@ __host__ __device__ __forceinline__ void group_coords(int64_t lid, int64_t tiles
   ta = r / gsize;
 }
 
-// The same in 32-bit arithmetic, for the W4 kernel's one tile per workgroup (tile counts < 2^31).
-__device__ __forceinline__ void tile_coords(uint32_t tiles_a, uint32_t tiles_b, uint32_t& ta, uint32_t& tb) {
-  const uint32_t lid = (uint32_t)xcd_remap(blockIdx.x, tiles_a * tiles_b);   // the grid is one workgroup per tile
-  constexpr uint32_t GB = 8;
+// The same in 32-bit arithmetic (tile counts < 2^31).
+__device__ __forceinline__ void group_coords32(uint32_t lid, uint32_t tiles_a, uint32_t tiles_b, uint32_t GB,
+                                               uint32_t& ta, uint32_t& tb) {
   const uint32_t in_group = GB * tiles_a;
   const uint32_t g = lid / in_group;
   const uint32_t first_b = g * GB;
@@ -140,6 +139,11 @@ __device__ __forceinline__ void tile_coords(uint32_t tiles_a, uint32_t tiles_b, 
   const uint32_t r = lid - g * in_group;
   tb = first_b + r % gsize;
   ta = r / gsize;
+}
+
+// For the W4 kernel, whose grid is one workgroup per tile.
+__device__ __forceinline__ void tile_coords(uint32_t tiles_a, uint32_t tiles_b, uint32_t& ta, uint32_t& tb) {
+  group_coords32((uint32_t)xcd_remap(blockIdx.x, tiles_a * tiles_b), tiles_a, tiles_b, 8, ta, tb);
 }
 
 __device__ __forceinline__ v4i frag(const uint8_t* s, int row, int chunk) {
@@ -1018,21 +1022,22 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
 // ---------------------------------------------------------------------------------------------------------
 // The fixup of a split launch: the pieces of each remainder tile added in slice order, then the tile kernel's
 // epilogue on the sums, element for element the same arithmetic (so W8 outputs equal the unsplit launch's bit for
-// bit).  Bound by reading the pieces (s x 256 KB a T256 tile): 72 tiles of 3 pieces (57 MB) take 14.6 us for the
-// input gradient and 18.7 us for W8A8.  A wave owns one column of 32 x 32 blocks (the NA blocks a tile-kernel wave
-// holds for one of its B-blocks: 32 output rows x ARW columns), FIX_WAVES waves a workgroup, so the launches that
-// split (48-128 tiles) spread over every CU; a workgroup per tile, as part of the tile kernel, took 19.5 us for the
-// same W8A8 pieces and knew no segments.  Two slices in flight per wave (registers) and tiles fixed up on the XCD
-// that ran their pieces were 0-37 % slower.  The LoRA factors come straight from global memory, the next 16-rank
-// chunk's loads in flight while this one is multiplied; the bf16 block goes through the wave's own LDS for
-// row-contiguous stores.
+// bit).  Bound by reading the pieces (s x 256 KB a T256 tile) on large launches, by latency on small ones.  A wave owns
+// one column of 32 x 32 blocks (the NA blocks a tile-kernel wave holds for one of its B-blocks: 32 output rows x ARW
+// columns), FIX_WAVES waves a workgroup, so the launches that split spread over every CU; a workgroup per tile, as
+// part of the tile kernel, knew no segments and took 19.5 us for 72 W8A8 tiles of 3 pieces (57 MB), this 14.0.
+// UMAX slices are in flight per wave: 4 (T128) or 2 (T256) where the launch leaves CUs idle (103 x 2560 -> 1024 with 4
+// pieces 18.8 -> 13.0 us, 14.7 before), one where it fills them (two there: 14.0 -> 18.1 us, fewer waves).  Tiles
+// fixed up on the XCD that ran their pieces were up to 37 % slower.  The LoRA factors come straight from global
+// memory, the next 16-rank chunk's loads in flight while this one is multiplied; the bf16 block goes through the
+// wave's own LDS for row-contiguous stores.
 // ---------------------------------------------------------------------------------------------------------
 constexpr int FIX_WAVES = 2;
 template <class C>
 constexpr int fix_wgs_per_tile() { return GW * C::NB / FIX_WAVES; }
 
-template <int EPI, class C, int NS>
-__global__ __launch_bounds__(64 * FIX_WAVES) void gemm_fixup_kernel(GemmArgsN<NS> p0) {
+template <int EPI, class C, int NS, int UMAX>
+__global__ __launch_bounds__(64 * FIX_WAVES, UMAX > 1 ? 1 : 2) void gemm_fixup_kernel(GemmArgsN<NS> p0) {
   constexpr bool BF16 = (EPI == EPI_DX || EPI == EPI_LIN || EPI == EPI_DXLIN);
   constexpr bool SCALED = (EPI == EPI_W8 || EPI == EPI_LIN);
   constexpr bool RA_T = (EPI == EPI_DX || EPI == EPI_DXLIN);
@@ -1047,13 +1052,13 @@ __global__ __launch_bounds__(64 * FIX_WAVES) void gemm_fixup_kernel(GemmArgsN<NS
   const int wa = w % C::WVA, wb = w / C::WVA;
   const int h = lane >> 5, c32 = lane & 31;
 
-  const int64_t tiles_a = (p0.rows_a + C::TA - 1) / C::TA, tiles_b = (p0.rows_b + C::TB - 1) / C::TB;
-  int64_t ta, tb;
-  group_coords(p0.dp_tiles + rt, tiles_a, tiles_b, p0.gb > 0 ? p0.gb : 8, ta, tb);
-  int64_t A0 = ta * C::TA;
+  uint32_t ta, tb;
+  group_coords32((uint32_t)(p0.dp_tiles + rt), (uint32_t)((p0.rows_a + C::TA - 1) / C::TA),
+                 (uint32_t)((p0.rows_b + C::TB - 1) / C::TB), p0.gb > 0 ? p0.gb : 8, ta, tb);
+  int64_t A0 = (int64_t)ta * C::TA;
   GemmBase p = p0;
   if constexpr (EPI == EPI_W8 && NS > 0) pick_segment(p0, p, A0);
-  const int64_t a0 = A0 + C::ARW * wa, b0 = tb * C::TB + C::BRW * wb + 32 * ib;
+  const int64_t a0 = A0 + C::ARW * wa, b0 = (int64_t)tb * C::TB + C::BRW * wb + 32 * ib;
   if (a0 >= p.rows_a || b0 >= p.rows_b) return;   // no barriers below: a wave past the matrix leaves
 
   const int64_t rb = b0 + c32 < p.rows_b ? b0 + c32 : p.rows_b - 1;   // this lane's B-row
@@ -1093,22 +1098,39 @@ __global__ __launch_bounds__(64 * FIX_WAVES) void gemm_fixup_kernel(GemmArgsN<NS
   constexpr int64_t PIECE_BYTES = (int64_t)C::TA * C::TB * 4;
   const uint32_t toff = 16u * (uint32_t)(64 * w + lane);
   if (lora) load_factors(0);
-  for (int sl = 0; sl < p.sk_s; ++sl) {
-    const uint8_t* pc = reinterpret_cast<const uint8_t*>(p.part) + ((int64_t)sl * p.sk_rem + rt) * PIECE_BYTES;
-    v4i q[NA][4];
+  // Slices sl .. sl + U - 1: all their loads are issued before the first is added (in slice order).
+  auto add_slices = [&](int sl, auto UC) {
+    constexpr int U = decltype(UC)::value;
+    v4i q[U][NA][4];
 #pragma unroll
-    for (int ia = 0; ia < NA; ++ia)
+    for (int u = 0; u < U; ++u) {
+      const uint8_t* pc = reinterpret_cast<const uint8_t*>(p.part) + ((int64_t)(sl + u) * p.sk_rem + rt) * PIECE_BYTES;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        q[ia][j] = *reinterpret_cast<const v4i*>(pc + (int64_t)((ia * NB + ib) * 4 + j) * GT * 16 + toff);
+      for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
-    for (int ia = 0; ia < NA; ++ia) {
-      const v16i v = __builtin_shufflevector(__builtin_shufflevector(q[ia][0], q[ia][1], 0, 1, 2, 3, 4, 5, 6, 7),
-                                             __builtin_shufflevector(q[ia][2], q[ia][3], 0, 1, 2, 3, 4, 5, 6, 7), 0, 1,
-                                             2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-      acc[ia] += __builtin_bit_cast(Acc, v);
+        for (int j = 0; j < 4; ++j)
+          q[u][ia][j] = *reinterpret_cast<const v4i*>(pc + (int64_t)((ia * NB + ib) * 4 + j) * GT * 16 + toff);
     }
+    __builtin_amdgcn_sched_barrier(0);   // or the scheduler sinks each load to its add, one latency after another
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int ia = 0; ia < NA; ++ia) {
+        const v16i v =
+            __builtin_shufflevector(__builtin_shufflevector(q[u][ia][0], q[u][ia][1], 0, 1, 2, 3, 4, 5, 6, 7),
+                                    __builtin_shufflevector(q[u][ia][2], q[u][ia][3], 0, 1, 2, 3, 4, 5, 6, 7), 0, 1, 2,
+                                    3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+        acc[ia] += __builtin_bit_cast(Acc, v);
+      }
+  };
+  int sl = 0;
+  if constexpr (UMAX >= 4) {
+    for (; sl + 4 <= p.sk_s; sl += 4) add_slices(sl, std::integral_constant<int, 4>{});
   }
+  if constexpr (UMAX >= 2) {
+    for (; sl + 2 <= p.sk_s; sl += 2) add_slices(sl, std::integral_constant<int, 2>{});
+  }
+  for (; sl < p.sk_s; ++sl) add_slices(sl, std::integral_constant<int, 1>{});
 
   if constexpr (EPI == EPI_ACC) {
     int32_t* out = static_cast<int32_t*>(p.out);
@@ -1467,15 +1489,26 @@ __global__ __launch_bounds__(256) void w4_fixup_kernel(W4Args p) {
   if (B0 >= p.M) return;
   v16f accf[1] = {v16f{0.f}};
   const float* src = p.part + (int64_t)blockIdx.x * (W4_BA * C::BB) + (4 * ib * 256 + (int)threadIdx.x) * 4;
-  for (int sl = 0; sl < p.s; ++sl) {
+  const int64_t stride = tiles * (W4_BA * C::BB);
+  auto add_slices = [&](int sl, auto UC) {   // U slices' loads issued before the first is added
+    constexpr int U = decltype(UC)::value;
+    v4f v[U][4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const v4f v = *reinterpret_cast<const v4f*>(src + q * 1024);
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) accf[0][4 * q + i] += v[i];
-    }
-    src += tiles * (W4_BA * C::BB);
-  }
+      for (int q = 0; q < 4; ++q) v[u][q] = *reinterpret_cast<const v4f*>(src + (sl + u) * stride + q * 1024);
+    __builtin_amdgcn_sched_barrier(0);   // or the scheduler sinks each load to its add
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) accf[0][4 * q + i] += v[u][q][i];
+  };
+  int sl = 0;
+  for (; sl + 4 <= p.s; sl += 4) add_slices(sl, std::integral_constant<int, 4>{});
+  for (; sl + 2 <= p.s; sl += 2) add_slices(sl, std::integral_constant<int, 2>{});
+  if (sl < p.s) add_slices(sl, std::integral_constant<int, 1>{});
   w4_epilogue<EPI, 1>(p, accf, A0, B0, smem);
 }
 
@@ -1565,14 +1598,15 @@ int launch_w4(W4Args p, void* ws, int64_t ws_bytes, hipStream_t st) {
 //   launch + rounds x (stages x stage cost + epilogue),
 // a round being CUs x workgroups-per-CU tiles, and the last, partly filled round (its tiles the remainder) either
 // run like the others or cut along the reduction into s pieces per tile, whose accumulators a fixup launch adds:
-//   ceil(stages / s) x stage cost + piece cost + 0.207 us per MB of pieces.
+//   ceil(stages / s) x stage cost + piece cost + 0.143 s + 0.239 us per MB of pieces (+ 11 us where full rounds run
+//   beside it: three launches, each with a tail of its own).
 // A stage (128 reduction bytes) of a partly filled round is cheaper (less contention for L2 and HBM, and a higher
 // clock), and dearer the more of the staged bytes no other tile shares: its cost is scaled by (alpha + (1 - alpha)
 // fill) (1 + m unique), unique = the operands' rows over the rows that the tiles stage.  The constants are fitted
-// to the measured times of every shape and split at 252 launches (int8 and bf16, M 96-4608, outputs 1536-32768,
-// reductions 1024-32768): the plan taken is on average 1.1 % from the fastest measured one, where the estimate it
-// replaced, fitted to full rounds, was 3.8 % (and 20-38 % on one-round launches of 256 x 256 tiles and on long
-// reductions over few tiles: the 768-token input gradient to 16384 columns 196.6 -> 164.8 us, 512 x 6144 over 16384
+// to the measured times of every shape and split at 552 launches (int8 and bf16, M 9-16896, outputs 512-32768,
+// reductions 512-32768), launches over 150 us with four times the weight; on 60 drawn launches beside those the plan
+// taken is on average 1.5 % from the fastest measured one and 8 % faster than the estimate it replaced, which was
+// fitted to full rounds (the 768-token input gradient to 16384 columns 196.6 -> 164.8 us, 512 x 6144 over 16384
 // 157.4 -> 114.0).
 struct SplitPlan {
   int64_t dp_tiles;   // tiles run over the full reduction
@@ -1586,10 +1620,10 @@ struct TileCost {
   double epi, piece;      // epilogue; piece ramp and store, fixup launch (0: the shape does not split)
 };
 constexpr TileCost TILE_COSTS[TILE_COUNT] = {
-    {256, 256, 1, 1.466, 1.466, 6.694, 10.84},
-    {256, 320, 1, 1.663, 1.663, 10.847, 0.0},
-    {192, 256, 1, 1.203, 1.203, 5.598, 0.0},
-    {128, 128, 2, 0.605, 0.989, 5.438, 9.167},
+    {256, 256, 1, 1.623, 1.623, 5.590, 7.418},
+    {256, 320, 1, 1.917, 1.917, 8.060, 0.0},
+    {192, 256, 1, 1.378, 1.378, 4.046, 0.0},
+    {128, 128, 2, 0.722, 1.010, 3.243, 5.165},
 };
 
 // Shortest segmented reduction that is cut (stages).  Below it a launch takes under 60 us and a cut gains a few.
@@ -1601,22 +1635,23 @@ SplitPlan tile_plan(int t, bool bf16, int64_t rows_a, int64_t rows_b, int nst, i
   const int64_t tiles = ((rows_a + c.ta - 1) / c.ta) * ((rows_b + c.tb - 1) / c.tb);
   const int64_t slots = (int64_t)cus * c.wpc, full = tiles / slots, rem = tiles - full * slots;
   const double unique = (double)(rows_a + rows_b) / ((double)tiles * (c.ta + c.tb));
-  const double k = (bf16 ? 1.074 : 1.0) * (1.0 + 0.63 * unique), epi = c.epi * (bf16 ? 0.711 : 1.0);
+  const double k = 1.0 + 0.395 * unique, epi = c.epi * (bf16 ? 0.822 : 1.0);
   auto stage = [&](int64_t active) {
     if (active > cus) return k * (c.alone + (c.shared - c.alone) * (double)(active - cus) / (double)cus);
-    return k * c.alone * (0.582 + 0.418 * (double)active / (double)cus);
+    return k * c.alone * (0.527 + 0.473 * (double)active / (double)cus);
   };
-  const double head = 1.069 + (double)full * (nst * stage(slots) + epi);
+  const double head = 1.525 + (double)full * (nst * stage(slots) + epi);
   SplitPlan q{tiles, 0, 1, head + (rem ? nst * stage(rem) + epi : 0.0)};
   if (can_split && c.piece > 0.0 && rem > 0) {
     for (int s = 2; s <= 10 && rem * s <= slots && nst / s >= 4; ++s) {
       const double mb = (double)(rem * s) * c.ta * c.tb * 4e-6;
-      const double t_s = head + (double)((nst + s - 1) / s) * stage(rem * s) + c.piece + 0.207 * mb;
+      const double t_s = head + (full ? 11.16 : 0.0) + (double)((nst + s - 1) / s) * stage(rem * s) + c.piece +
+                         0.143 * s + 0.239 * mb;
       if (t_s < q.cost) q = SplitPlan{full * slots, (int)rem, s, t_s};
     }
   }
-  // no plan is faster than reading the operands once (5 TB/s)
-  const double floor_us = 3.069 + (double)(rows_a + rows_b) * nst * WBK / 5e6;
+  // no plan is faster than reading the operands once (6 TB/s)
+  const double floor_us = 1.525 + (double)(rows_a + rows_b) * nst * WBK / 6e6;
   if (q.cost < floor_us) q.cost = floor_us;
   return q;
 }
@@ -1733,8 +1768,11 @@ int launch_split_as(const GemmArgs& p, const SplitPlan& q, hipStream_t st) {
   else pf = slim(p);
   hipLaunchKernelGGL((gemm_nt_kernel<EPI, MODE, C, NS>), dim3((unsigned)(q.rem * q.s)), dim3(GT), C::LDS, st, ps);
   if (q.dp_tiles > 0 && (rc = launch_full<EPI, C>(p, st))) return rc;
-  hipLaunchKernelGGL((gemm_fixup_kernel<EPI, C, FNS>), dim3((unsigned)(q.rem * fix_wgs_per_tile<C>())),
-                     dim3(64 * FIX_WAVES), 0, st, pf);
+  const dim3 grid((unsigned)(q.rem * fix_wgs_per_tile<C>())), block(64 * FIX_WAVES);
+  // several slices in flight where the launch leaves CUs idle, one (fewer registers, more waves) where it fills them
+  constexpr int U = C::NA <= 2 ? 4 : 2;
+  if ((int)grid.x <= 2 * k2q_cu_count()) hipLaunchKernelGGL((gemm_fixup_kernel<EPI, C, FNS, U>), grid, block, 0, st, pf);
+  else hipLaunchKernelGGL((gemm_fixup_kernel<EPI, C, FNS, 1>), grid, block, 0, st, pf);
   return K2Q_OK;
 }
 

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,K,Ns,r", [(9, 6144, (512, 256), 16), (129, 16384, (256, 256, 512), 48),
-                                      (768, 6144, (16384, 16384), 16), (1300, 6144, (6144, 1536, 1536, 6144), 0),
+                                      (1000, 6144, (9216, 9216), 16), (1000, 12288, (1536, 512, 1024, 1536), 0),
                                       (300, 6144, (1536, 1536, 1536), 16)])
 def test_grouped_split_equals_separate(k2, dev, M, K, Ns, r):
     L = k2._lib
