@@ -304,12 +304,12 @@ class _SiblingGroup:
 
     def _a_stack(self, As):
         """The members' A factors stacked along the rank.  Kept while every factor is the adapter's own
-        parameter (a leaf the module holds, so its object, version and pointer identify its values: an optimizer
+        parameter (the module holds it, so its object, version and pointer identify its values: an optimizer
         step or a re-pointed parameter rebuilds the stack); padded or converted factors are new tensors every
-        call and are stacked every call."""
+        call, whose object and memory the next call's may take over, and are stacked every call."""
         if not As:
             return None
-        if not all(a.is_leaf for a in As):
+        if not all(isinstance(a, nn.Parameter) for a in As):
             with torch.no_grad():
                 return torch.cat(As) if len(As) > 1 else As[0].detach()
         key = tuple((id(a), a._version, a.data_ptr(), a.device) for a in As)
