@@ -100,6 +100,12 @@ int64_t k2q_lora_down_ws_bytes(int64_t M, int64_t K, int64_t r);
 int k2q_lora_down(const uint16_t* x, int64_t M, int64_t K, int64_t ldx, const float* lora_a, int64_t r,
                   void* ws, int64_t ws_bytes, float* u, void* stream);
 
+/* Both factors of an adapter padded with zero ranks to a rank the kernels take, in one launch (no counterpart in the
+ * reference): ap (rp x K) = a (r x K) and zero rows, bp (N x rp) = b (N x r) and zero columns.  rp % 16 == 0,
+ * K % 4 == 0. */
+int k2q_pad_factors(const float* a, const float* b, int64_t r, int64_t rp, int64_t K, int64_t N, float* ap, float* bp,
+                    void* stream);
+
 /* LoRA gradients through the frozen base (the autograd of lora.py:47-48):
  *   g = scale * dy @ lora_b (M x r), dA = g^T x (r x K), dB = scale * dy^T u (N x r),
  * all f32 from bf16 dy (M x N) / x (M x K) and f32 u (M x r) / lora_b (N x r).  dA / dB nullable (x / u

@@ -70,6 +70,7 @@ _SIGNATURES = {
     "k2q_rmsmod_bwd": ([_p, _p, _i64, _i64, _p, _f32, _p, _i64, _i64, _p, _p], _int),
     "k2q_lora_down_ws_bytes": ([_i64, _i64, _i64], _i64),
     "k2q_lora_down": ([_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p], _int),
+    "k2q_pad_factors": ([_p, _p, _i64, _i64, _i64, _i64, _p, _p, _p], _int),
     "k2q_lora_grads_ws_bytes": ([_i64, _i64, _i64, _i64], _i64),
     "k2q_lora_grads": ([_p, _p, _p, _p, _i64, _f32, _i64, _i64, _i64, _p, _p, _p, _p, _i64, _p], _int),
     "k2q_lora_grads_grouped_ws_bytes": ([_p, _i64, _i64, _i64, _i64], _i64),
@@ -445,6 +446,23 @@ def _check_lora_down(x, A) -> None:
         raise ValueError(f"lora_A has in_features {A.shape[1]}, x has {x.shape[1]}")
     _check_rank(A.shape[0])
     _device_check(dev)
+
+
+def pad_factors(A: torch.Tensor, B: torch.Tensor, rp: int):
+    """``A`` (r,K) and ``B`` (N,r) f32 with zero ranks appended up to ``rp`` (one launch): ``((rp,K), (N,rp))``."""
+    r = _fast().pad_factors(A, B, rp)
+    if r.__class__ is tuple:
+        return r
+    return _refused(r, "k2q_pad_factors", lambda: _native.pad_factors(A, B, rp), lambda: _check_pad_factors(A, B, rp))
+
+
+def _check_pad_factors(A, B, rp: int) -> None:
+    _need(A, "lora_A", torch.float32, 2)
+    _need(B, "lora_B", torch.float32, 2, A.device)
+    if B.shape[1] != A.shape[0] or rp < A.shape[0] or A.shape[1] % 4:
+        raise ValueError(f"lora_A {tuple(A.shape)} / lora_B {tuple(B.shape)} cannot be padded to rank {rp}")
+    _check_rank(rp)
+    _device_check(A.device)
 
 
 def lora_grads(dy, x, u, lora_b, lora_scale: float):

@@ -26,6 +26,7 @@ struct Api {
   decltype(&k2q_lora_grads_ws_bytes) lora_grads_ws_bytes;
   decltype(&k2q_lora_down) lora_down;
   decltype(&k2q_lora_down_ws_bytes) lora_down_ws_bytes;
+  decltype(&k2q_pad_factors) pad_factors;
   decltype(&k2q_dx_prep_eff) dx_prep_eff;
   decltype(&k2q_gemm_dx_lin) gemm_dx_lin;
   decltype(&k2q_gemm_dx_ws_bytes) gemm_dx_ws_bytes;
@@ -247,6 +248,30 @@ PyObject* py_lora_down(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// pad_factors(A, B, rp) -> (rp, K) and (N, rp) with zero ranks behind A's and B's
+PyObject* py_pad_factors(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  K2Q_ARGS(3)
+  return guarded([&]() -> PyObject* {
+    const Tensor *A = tensor_of(a[0], bad), *B = tensor_of(a[1], bad);
+    const int64_t rp = PyLong_AsLongLong(a[2]);
+    if (PyErr_Occurred()) return nullptr;
+    if (bad || !A || !B) K2Q_REFUSE;
+    const c10::Device d = A->device();
+    if (!ready(d) || !operand(A, at::kFloat, 2, d) || !operand(B, at::kFloat, 2, d)) K2Q_REFUSE;
+    const int64_t r = A->size(0), K = A->size(1), N = B->size(0);
+    if (B->size(1) != r || r < 1 || rp < r || !rank_ok(rp) || K % 4 || K < 4 || N < 1) K2Q_REFUSE;
+    void* st;
+    if (!stream_of(d, st)) return nullptr;
+    Tensor ap = alloc({rp, K}, at::kFloat, d), bp = alloc({N, rp}, at::kFloat, d);
+    const int rc = foreign([&] {
+      return api.pad_factors(as<float>(ptr(A)), as<float>(ptr(B)), r, rp, K, N, as<float>(ptr(ap)), as<float>(ptr(bp)),
+                             st);
+    });
+    if (rc) return PyLong_FromLong(rc);
+    return pack({ap, bp});
+  });
+}
+
 // A ConvRot layer's codes and scales on device d; N, K its widths.
 bool convrot_ok(const Tensor* q, const Tensor* s, bool w4, c10::Device d, int64_t& N, int64_t& K) {
   if (!operand(q, w4 ? at::kByte : at::kChar, 2, d) || !operand(s, w4 ? at::kBFloat16 : at::kFloat, w4 ? 2 : 1, d))
@@ -398,7 +423,8 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!get("k2q_linear_fwd", api.linear_fwd) || !get("k2q_linear_fwd_ws_bytes", api.linear_fwd_ws_bytes) ||
       !get("k2q_linear_fwd_fuses_down", api.linear_fwd_fuses_down) || !get("k2q_lora_grads", api.lora_grads) ||
       !get("k2q_lora_grads_ws_bytes", api.lora_grads_ws_bytes) || !get("k2q_lora_down", api.lora_down) ||
-      !get("k2q_lora_down_ws_bytes", api.lora_down_ws_bytes) || !get("k2q_dx_prep_eff", api.dx_prep_eff) ||
+      !get("k2q_lora_down_ws_bytes", api.lora_down_ws_bytes) || !get("k2q_pad_factors", api.pad_factors) ||
+      !get("k2q_dx_prep_eff", api.dx_prep_eff) ||
       !get("k2q_gemm_dx_lin", api.gemm_dx_lin) || !get("k2q_gemm_dx_ws_bytes", api.gemm_dx_ws_bytes) ||
       !get("k2q_dequant_fp8", api.dequant_fp8) || !get("k2q_gemm_bf16", api.gemm_bf16) ||
       !get("k2q_gemm_bf16_ws_bytes", api.gemm_bf16_ws_bytes))
@@ -422,7 +448,7 @@ PyObject* py_device_checked(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {K2Q_METHOD(bind),        K2Q_METHOD(device_checked), K2Q_METHOD(alloc_codes),
                          K2Q_METHOD(linear_fwd),  K2Q_METHOD(lora_grads),     K2Q_METHOD(lora_down),
                          K2Q_METHOD(dx_weight),   K2Q_METHOD(gemm_dx),        K2Q_METHOD(dequant_fp8),
-                         K2Q_METHOD(gemm_bf16),   {nullptr, nullptr, 0, nullptr}};
+                         K2Q_METHOD(gemm_bf16),   K2Q_METHOD(pad_factors),    {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_k2q_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -639,6 +639,44 @@ int lora_down_impl(const uint16_t* x, int64_t M, int64_t K, int64_t ldx, const f
   return K2Q_OK;
 }
 
+namespace {
+
+// Both factors of an adapter at a rank the kernels take: ap (rp x K) = a with zero rows r .. rp-1, bp (N x rp) = b
+// with zero columns.  Four floats per thread; K % 4 == 0 and rp % 4 == 0, so a thread's four lie in one row.
+__global__ __launch_bounds__(256) void pad_factors_kernel(const float* __restrict__ a, const float* __restrict__ b,
+                                                          int r, int rp, int64_t K, int64_t N, float* __restrict__ ap,
+                                                          float* __restrict__ bp) {
+  const int64_t na = (int64_t)rp * K / 4, nb = N * rp / 4;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  v4f v = v4f{0.f, 0.f, 0.f, 0.f};
+  if (i < na) {
+    if (4 * i < (int64_t)r * K) v = *reinterpret_cast<const v4f*>(a + 4 * i);
+    *reinterpret_cast<v4f*>(ap + 4 * i) = v;
+    return;
+  }
+  i -= na;
+  if (i >= nb) return;
+  const int64_t n = 4 * i / rp;
+  const int j = (int)(4 * i - n * rp);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (j + e < r) v[e] = b[n * r + j + e];
+  *reinterpret_cast<v4f*>(bp + 4 * i) = v;
+}
+
+}  // namespace
+
+extern "C" int k2q_pad_factors(const float* a, const float* b, int64_t r, int64_t rp, int64_t K, int64_t N, float* ap,
+                               float* bp, void* stream) {
+  if (!a || !b || !ap || !bp || r < 1 || rp < r || !rank_ok(rp) || K < 4 || K % 4 || N < 1) return K2Q_EINVAL;
+  if (!k2q_aligned(a, 16) || !k2q_aligned(b, 4) || !k2q_aligned(ap, 16) || !k2q_aligned(bp, 16)) return K2Q_EINVAL;
+  const int64_t blocks = ((rp * K + N * rp) / 4 + 255) / 256;
+  if (blocks > 0x7fffffff) return K2Q_EUNSUPPORTED;
+  hipLaunchKernelGGL(pad_factors_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), a, b,
+                     (int)r, (int)rp, K, N, ap, bp);
+  return k2q_launch_status();
+}
+
 extern "C" int k2q_dx_prep_eff(const int8_t* qw, const float* sw, const uint8_t* qw4, const uint16_t* sw4,
                                int64_t N, int64_t K, uint16_t* wt, void* stream) {
   const bool w4 = qw4 != nullptr;

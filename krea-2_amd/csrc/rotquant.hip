@@ -1,8 +1,7 @@
 // Kernel (1): block Walsh-Hadamard rotation + per-row int8 quantization (and the int4 group-64 weight
 // quantizer), one HBM pass.
 //
-// Spec (no reference code exists for it): BASELINE.json north_star kernel (1); the absmax floor mirrors
-// reference quantize.py:36.  Arithmetic, fixed so the int8 codes are bit-exact:
+// The reference has no code for it; the absmax floor mirrors reference quantize.py:36.  Arithmetic, fixed so the int8 codes are bit-exact:
 //   * FWHT of every 128-wide block, float32, unnormalised, radix-2 butterfly with stage strides
 //     1, 2, 4, ..., 64 in that order; the pair (i, i+s) becomes (a+b, a-b).
 //   * absmax over the whole rotated row, floored at 1e-8; inv = 127/absmax and s = absmax/127, each one

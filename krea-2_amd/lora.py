@@ -52,8 +52,21 @@ def _is_adaptable(mod) -> bool:
     return isinstance(mod, nn.Linear) or bool(getattr(mod, "is_quant_linear", False))
 
 
-def _padded_rank(rank: int) -> int:
-    return -(-rank // _lib.RANK_ALIGN) * _lib.RANK_ALIGN
+class _PadRank(torch.autograd.Function):
+    """``F.pad`` of both factors with zero ranks, in one launch (``k2q_pad_factors``) and one node: F.pad fills and
+    copies each factor on its own.  The gradients drop the padded ranks.  Rank 8 at 333 x 3072 -> 3072: forward 46 ->
+    32.5 us, forward and backward 201 -> 174 us; rank 24 at 768 x 6144 -> 6144 (W4A8), both ways 199 -> 192 us."""
+
+    @staticmethod
+    def forward(ctx, A, B, rp):
+        ctx.rank = A.shape[0]
+        ctx.set_materialize_grads(False)
+        return _lib.pad_factors(A, B, rp)
+
+    @staticmethod
+    def backward(ctx, dA, dB):
+        r = ctx.rank
+        return (None if dA is None else dA[:r].contiguous(), None if dB is None else dB[:, :r].contiguous(), None)
 
 
 class LoRALinear(nn.Module):
@@ -86,11 +99,15 @@ class LoRALinear(nn.Module):
         A, B = self.lora_A, self.lora_B
         if A.dtype != torch.float32:
             A, B = A.float(), B.float()
+        A, B = A.contiguous(), B.contiguous()
         extra = -self.rank % _lib.RANK_ALIGN
-        if extra:
-            A = F.pad(A, (0, 0, 0, extra))
-            B = F.pad(B, (0, extra))
-        return A.contiguous(), B.contiguous()
+        if not extra:
+            return A, B
+        if A.is_cuda and A.data_ptr() % 16 == 0 and B.data_ptr() % 16 == 0:
+            if torch.is_grad_enabled() and (A.requires_grad or B.requires_grad):
+                return _PadRank.apply(A, B, self.rank + extra)
+            return _lib.pad_factors(A, B, self.rank + extra)
+        return F.pad(A, (0, 0, 0, extra)), F.pad(B, (0, extra))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         s = self.scale * self.scale_mul
