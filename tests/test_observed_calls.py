@@ -1,0 +1,42 @@
+"""CPU tests: a call without gradients skips its autograd node only where nobody looks on.  A tracer has to find the
+node in its graph (a library call's result would be a constant there), and a tangent has to be refused, not dropped."""
+import pytest
+import torch
+from torch.autograd import forward_ad
+
+
+@pytest.fixture
+def layer(k2, monkeypatch):
+    """An fp8 layer whose library calls work on the tensors' values, seen by no tracer and carrying no tangents."""
+    def forward(x, A, B, q, s, bias, scale):
+        w = torch.tensor(q.float().tolist()) * s.float().view(-1, 1)
+        return torch.tensor((torch.tensor(x.float().tolist()) @ w.t()).tolist(), dtype=torch.bfloat16), None
+
+    monkeypatch.setattr(k2.quantize, "_fp8_forward", forward)
+    g = torch.Generator().manual_seed(1)
+    q = torch.randn(128, 128, generator=g).to(torch.float8_e4m3fn)
+    return k2.Fp8Linear.from_quantized(q, torch.ones(128, dtype=torch.bfloat16), None)
+
+
+def test_trace_follows_its_input(layer):
+    x, other = torch.randn(2, 4, 128).to(torch.bfloat16)
+    with torch.no_grad():
+        traced = torch.jit.trace(layer, x, check_trace=False)
+        assert torch.equal(traced(other), layer(other))
+
+
+def test_tangents_are_refused(layer):
+    x = torch.randn(4, 128).to(torch.bfloat16)
+    with torch.no_grad():
+        layer(x)
+        with forward_ad.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+            layer(forward_ad.make_dual(x, torch.ones_like(x)))
+
+
+def test_padding_under_a_tracer_or_a_dual_level_is_torch_operations(k2):
+    assert not k2._lib.observed()
+    with forward_ad.dual_level():
+        assert k2._lib.observed()
+    seen = []
+    torch.jit.trace(lambda t: (seen.append(k2._lib.observed()), t + 1)[1], torch.zeros(2), check_trace=False)
+    assert seen == [True]
