@@ -32,6 +32,16 @@ def _rows(t: torch.Tensor, K: int) -> torch.Tensor:
     return t2
 
 
+def _dense_grad(dh, like):
+    """A producer's output gradient as the kernels read it: contiguous bf16, zeros where autograd has none.  Its node
+    takes undefined gradients as None: autograd would otherwise write zeros for the codes and scales too, which have
+    no gradient (two fills per producer: an MLP half's training pass at 768 x 6144 x 16384 1070.3 -> 1064.6 us)."""
+    if dh is None:
+        return torch.zeros(like.shape, dtype=torch.bfloat16, device=like.device)
+    dh = dh.contiguous()
+    return dh if dh.dtype == torch.bfloat16 else dh.to(torch.bfloat16)
+
+
 class _SwiGLUQuantFn(torch.autograd.Function):
     """Forward ``h = bf16(bf16(silu(g)) * u)`` (``mmdit.py:178``) with the codes of ``h``; backward
     ``k2q_swiglu_bwd`` (the autograd of the two eager bf16 ops)."""
@@ -41,14 +51,13 @@ class _SwiGLUQuantFn(torch.autograd.Function):
         h, q, s = _lib.swiglu_rotquant(g2, u2)
         ctx.save_for_backward(g2, u2)
         ctx.mark_non_differentiable(q, s)
+        ctx.set_materialize_grads(False)
         return h, q, s
 
     @staticmethod
     def backward(ctx, dh, _dq, _ds):
         g2, u2 = ctx.saved_tensors
-        dh = dh.contiguous()
-        if dh.dtype != torch.bfloat16:
-            dh = dh.to(torch.bfloat16)
+        dh = _dense_grad(dh, g2)
         g2, u2 = g2.contiguous(), u2.contiguous()
         dg, du = _lib.swiglu_bwd(dh, g2, u2)
         return dg, du
@@ -80,6 +89,7 @@ class _RmsModQuantFn(torch.autograd.Function):
         ctx.eps, ctx.rpb = eps, rows_per_batch
         ctx.save_for_backward(x2, norm_scale, mod_scale, mod_shift)
         ctx.mark_non_differentiable(q, s)
+        ctx.set_materialize_grads(False)
         return h, q, s
 
     @staticmethod
@@ -89,9 +99,7 @@ class _RmsModQuantFn(torch.autograd.Function):
             return None, None, None, None, None, None
         M = x2.shape[0]
         rpb = ctx.rpb if ms.shape[0] > 1 else M
-        dh = dh.contiguous()
-        if dh.dtype != torch.bfloat16:
-            dh = dh.to(torch.bfloat16)
+        dh = _dense_grad(dh, x2)
         dx = _lib.rmsmod_bwd(dh, x2.contiguous(), ns, ctx.eps, ms, rpb)
         return dx, None, None, None, None, None
 
