@@ -117,11 +117,20 @@ PyObject* guarded(F&& f) {
   return nullptr;
 }
 
-template <class F>
-int foreign(F&& f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS rc = f();
-  Py_END_ALLOW_THREADS return rc;
+template <class T>
+struct Plain {
+  using type = T;   // an argument of this type is converted to it, not deduced from
+};
+
+// Calls an entry point with the GIL released.  The arguments are values made before that: reading a tensor's pointer can
+// throw (a functorch wrapper has none), and nothing may throw without the GIL.
+template <class... P>
+int foreign(int (*fn)(P...), typename Plain<P>::type... args) {
+  struct Released {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return fn(args...);
 }
 
 #define K2Q_ARGS(N)                                                       \
@@ -181,12 +190,10 @@ PyObject* py_linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
         api.linear_fwd_ws_bytes(wmode, M, N, K, 0) == 0)
       nws = 0;
     Tensor ws = workspace(nws, d);
-    const int rc = foreign([&] {
-      return api.linear_fwd(as<uint16_t>(ptr(x)), x->stride(0), M, K, as<int8_t>(ptr(qx)), as<float>(ptr(sx)),
-                            ready_codes, as<float>(ptr(A)), as<float>(A ? ptr(B) : nullptr), r, (float)scale,
-                            as<float>(ptr(u)), wmode, ptr(qw), ptr(sw), as<float>(ptr(bias)), N, as<uint16_t>(ptr(y)),
-                            ptr(ws), nws, st);
-    });
+    const int rc = foreign(api.linear_fwd, as<uint16_t>(ptr(x)), x->stride(0), M, K, as<int8_t>(ptr(qx)),
+                           as<float>(ptr(sx)), ready_codes, as<float>(ptr(A)), as<float>(A ? ptr(B) : nullptr), r,
+                           (float)scale, as<float>(ptr(u)), wmode, ptr(qw), ptr(sw), as<float>(ptr(bias)), N,
+                           as<uint16_t>(ptr(y)), ptr(ws), nws, st);
     if (rc) return PyLong_FromLong(rc);
     return pack({y, need_u ? u : Tensor()});
   });
@@ -217,11 +224,9 @@ PyObject* py_lora_grads(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor ws = workspace(nws, d);
     Tensor g = alloc({M, r}, at::kFloat, d);
     Tensor dA = x ? alloc({r, K}, at::kFloat, d) : Tensor(), dB = u ? alloc({N, r}, at::kFloat, d) : Tensor();
-    const int rc = foreign([&] {
-      return api.lora_grads(as<uint16_t>(ptr(dy)), as<uint16_t>(ptr(x)), as<float>(ptr(u)), as<float>(ptr(B)), r,
-                            (float)scale, M, N, K, as<float>(ptr(g)), as<float>(ptr(dA)), as<float>(ptr(dB)), ptr(ws),
-                            nws, st);
-    });
+    const int rc = foreign(api.lora_grads, as<uint16_t>(ptr(dy)), as<uint16_t>(ptr(x)), as<float>(ptr(u)),
+                           as<float>(ptr(B)), r, (float)scale, M, N, K, as<float>(ptr(g)), as<float>(ptr(dA)),
+                           as<float>(ptr(dB)), ptr(ws), nws, st);
     if (rc) return PyLong_FromLong(rc);
     return pack({g, dA, dB});
   });
@@ -241,9 +246,8 @@ PyObject* py_lora_down(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!stream_of(d, st)) return nullptr;
     const int64_t nws = api.lora_down_ws_bytes(M, K, r);
     Tensor ws = workspace(nws, d), u = alloc({M, r}, at::kFloat, d);
-    const int rc = foreign([&] {
-      return api.lora_down(as<uint16_t>(ptr(x)), M, K, K, as<float>(ptr(A)), r, ptr(ws), nws, as<float>(ptr(u)), st);
-    });
+    const int rc = foreign(api.lora_down, as<uint16_t>(ptr(x)), M, K, K, as<float>(ptr(A)), r, ptr(ws), nws,
+                           as<float>(ptr(u)), st);
     return rc ? PyLong_FromLong(rc) : wrap(u);
   });
 }
@@ -263,10 +267,8 @@ PyObject* py_pad_factors(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* st;
     if (!stream_of(d, st)) return nullptr;
     Tensor ap = alloc({rp, K}, at::kFloat, d), bp = alloc({N, rp}, at::kFloat, d);
-    const int rc = foreign([&] {
-      return api.pad_factors(as<float>(ptr(A)), as<float>(ptr(B)), r, rp, K, N, as<float>(ptr(ap)), as<float>(ptr(bp)),
-                             st);
-    });
+    const int rc = foreign(api.pad_factors, as<float>(ptr(A)), as<float>(ptr(B)), r, rp, K, N, as<float>(ptr(ap)),
+                           as<float>(ptr(bp)), st);
     if (rc) return PyLong_FromLong(rc);
     return pack({ap, bp});
   });
@@ -295,11 +297,9 @@ PyObject* py_dx_weight(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* st;
     if (!stream_of(d, st)) return nullptr;
     Tensor wt = alloc({K, N}, at::kBFloat16, d);
-    const int rc = foreign([&] {
-      return api.dx_prep_eff(w4 ? nullptr : as<int8_t>(ptr(q)), w4 ? nullptr : as<float>(ptr(s)),
-                             w4 ? as<uint8_t>(ptr(q)) : nullptr, w4 ? as<uint16_t>(ptr(s)) : nullptr, N, K,
-                             as<uint16_t>(ptr(wt)), st);
-    });
+    const int rc = foreign(api.dx_prep_eff, w4 ? nullptr : as<int8_t>(ptr(q)), w4 ? nullptr : as<float>(ptr(s)),
+                           w4 ? as<uint8_t>(ptr(q)) : nullptr, w4 ? as<uint16_t>(ptr(s)) : nullptr, N, K,
+                           as<uint16_t>(ptr(wt)), st);
     return rc ? PyLong_FromLong(rc) : wrap(wt);
   });
 }
@@ -311,10 +311,9 @@ PyObject* dx_lin(const Tensor& dy, const Tensor& wt, const Tensor* g, const Tens
   Tensor dx = alloc({M, K}, at::kBFloat16, d);
   const int64_t nws = api.gemm_dx_ws_bytes(M, N, K);
   Tensor ws = workspace(nws, d);
-  const int rc = foreign([&] {
-    return api.gemm_dx_lin(as<uint16_t>(dy.data_ptr()), as<uint16_t>(wt.data_ptr()), M, N, K, as<float>(ptr(g)),
-                           r ? as<float>(ptr(A)) : nullptr, r, as<uint16_t>(dx.data_ptr()), ptr(ws), nws, st);
-  });
+  const int rc = foreign(api.gemm_dx_lin, as<uint16_t>(dy.data_ptr()), as<uint16_t>(wt.data_ptr()), M, N, K,
+                         as<float>(ptr(g)), r ? as<float>(ptr(A)) : nullptr, r, as<uint16_t>(dx.data_ptr()), ptr(ws),
+                         nws, st);
   return rc ? PyLong_FromLong(rc) : wrap(dx);
 }
 
@@ -366,9 +365,8 @@ PyObject* py_dequant_fp8(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* st;
     if (!stream_of(d, st)) return nullptr;
     Tensor w = tr ? alloc({K, N}, at::kBFloat16, d) : alloc({N, K}, at::kBFloat16, d);
-    const int rc = foreign([&] {
-      return api.dequant_fp8(as<uint8_t>(ptr(q)), as<uint16_t>(ptr(s)), N, K, tr, as<uint16_t>(ptr(w)), st);
-    });
+    const int rc = foreign(api.dequant_fp8, as<uint8_t>(ptr(q)), as<uint16_t>(ptr(s)), N, K, tr, as<uint16_t>(ptr(w)),
+                           st);
     return rc ? PyLong_FromLong(rc) : wrap(w);
   });
 }
@@ -398,11 +396,9 @@ PyObject* py_gemm_bf16(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Tensor y = alloc({M, N}, at::kBFloat16, d);
     const int64_t nws = api.gemm_bf16_ws_bytes(M, N, K);
     Tensor ws = workspace(nws, d);
-    const int rc = foreign([&] {
-      return api.gemm_bf16(as<uint16_t>(ptr(x)), as<uint16_t>(ptr(w)), as<float>(ptr(bias)), as<float>(ptr(u)),
-                           u ? as<float>(ptr(B)) : nullptr, r, (float)scale, M, N, K, as<uint16_t>(ptr(y)), ptr(ws),
-                           nws, st);
-    });
+    const int rc = foreign(api.gemm_bf16, as<uint16_t>(ptr(x)), as<uint16_t>(ptr(w)), as<float>(ptr(bias)),
+                           as<float>(ptr(u)), u ? as<float>(ptr(B)) : nullptr, r, (float)scale, M, N, K,
+                           as<uint16_t>(ptr(y)), ptr(ws), nws, st);
     return rc ? PyLong_FromLong(rc) : wrap(y);
   });
 }

@@ -1,0 +1,48 @@
+"""CPU tests of the native wrappers' error paths: an operand without storage (a functorch wrapper) comes back as a Python
+exception, as it does from a ctypes call, whichever operand it is."""
+import subprocess
+import sys
+from pathlib import Path
+
+ROOT = Path(__file__).resolve().parents[1]
+
+# Fake GPU tensors pass the checks of shape, type and device (and read as null pointers, which the library refuses);
+# the operand under vmap is the one whose pointer cannot be read.
+_CHILD = """
+import sys
+sys.path.insert(0, ROOT)
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+import __graft_entry__ as ge
+k2 = ge.load_package()
+k2._lib._stream_of_index = lambda i: 0
+native = k2._lib._fast()
+native.device_checked(0)
+M, K, N, r = 16, 256, 128, 16
+with FakeTensorMode():
+    def t(*shape, dtype=torch.float32):
+        return torch.empty(shape, dtype=dtype, device="cuda:0")
+    ops = dict(x=t(M, K, dtype=torch.bfloat16), qx=t(M, K, dtype=torch.int8), sx=t(M), A=t(r, K), B=t(N, r),
+               qw=t(N, K, dtype=torch.int8), sw=t(N), bias=t(N))
+
+    for name, w in ops.items():
+        def call(wrapped):
+            o = dict(ops, **{name: wrapped})
+            native.linear_fwd(o["x"], o["qx"], o["sx"], False, o["A"], o["B"], 1.0, o["qw"], o["sw"], o["bias"], False,
+                              True)
+            return wrapped
+
+        try:
+            torch.func.vmap(call)(torch.empty((2, *w.shape), dtype=w.dtype, device="cuda:0"))
+        except RuntimeError as e:
+            assert "data pointer" in str(e), e
+            print("raised:", name, flush=True)
+"""
+
+
+def test_operand_without_storage_raises():
+    r = subprocess.run([sys.executable, "-c", _CHILD.replace("ROOT", repr(str(ROOT)))], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr[-2000:]
+    assert [line.split()[1] for line in r.stdout.splitlines() if line.startswith("raised:")] == \
+        ["x", "qx", "sx", "A", "B", "qw", "sw", "bias"]
