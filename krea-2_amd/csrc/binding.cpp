@@ -9,6 +9,7 @@
 // checked yet (the Python wrapper then runs the full checks, which name the argument, and calls again); or the entry
 // point's status as an int when it refuses the call.  Nothing is kept between calls but the entry points' addresses
 // and which devices are gfx950.  The GIL is released around the foreign calls.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -104,15 +105,14 @@ PyObject* pack(std::initializer_list<Tensor> ts) {
 bool rank_ok(int64_t r) { return r >= 16 && r <= K2Q_MAX_RANK && r % 16 == 0; }
 bool width_ok(int64_t k) { return k >= 128 && k % 128 == 0 && k <= 16384; }
 
-// Runs f with C++ exceptions turned into Python ones.
+// Runs f with C++ exceptions turned into the Python ones that torch's own bindings give (an allocation that fails is
+// torch.OutOfMemoryError, which callers catch by that name).
 template <class F>
 PyObject* guarded(F&& f) {
   try {
     return f();
-  } catch (const c10::Error& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (const std::exception&) {
+    torch::translate_exception_to_python(std::current_exception());
   }
   return nullptr;
 }

@@ -1,8 +1,13 @@
-"""CPU tests of the native wrappers' error paths: an operand without storage (a functorch wrapper) comes back as a Python
-exception, as it does from a ctypes call, whichever operand it is."""
+"""Tests of the native wrappers' error paths: an operand without storage (a functorch wrapper) comes back as a Python
+exception, as it does from a ctypes call, whichever operand it is, and an allocation that fails raises what torch.empty
+raises."""
 import subprocess
 import sys
 from pathlib import Path
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 ROOT = Path(__file__).resolve().parents[1]
 
@@ -46,3 +51,18 @@ def test_operand_without_storage_raises():
     assert r.returncode == 0, r.stdout + r.stderr[-2000:]
     assert [line.split()[1] for line in r.stdout.splitlines() if line.startswith("raised:")] == \
         ["x", "qx", "sx", "A", "B", "qw", "sw", "bias"]
+
+
+def test_failed_allocation_keeps_its_class(k2):
+    """A device that this build has no backend for is a NotImplementedError of torch's, not a plain RuntimeError."""
+    with FakeTensorMode():
+        x = torch.empty((4, 128), device="xpu:0")
+    with pytest.raises(NotImplementedError):
+        k2._lib.alloc_codes(x)
+
+
+@pytest.mark.gpu
+def test_out_of_memory_keeps_its_class(k2, dev):
+    x = torch.zeros((1, 128), dtype=torch.bfloat16, device=dev).expand(1 << 36, 128)     # codes of 8 TiB
+    with pytest.raises(torch.OutOfMemoryError):
+        k2._lib.alloc_codes(x)
