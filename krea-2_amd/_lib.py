@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import importlib.util
+import sysconfig
 import threading
 from pathlib import Path
 
@@ -130,13 +131,25 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def _running() -> str:
+    """The torch and Python builds that run, as ``build.py`` writes them into the extension."""
+    return f"torch {torch.__version__}, {sysconfig.get_config_var('SOABI')}"
+
+
 def _bind_native(lib) -> None:
     global _native
     if not NATIVE_PATH.exists():
         raise RuntimeError(f"{NATIVE_PATH} is not built; run krea-2_amd/build.py")
     spec = importlib.util.spec_from_file_location("_k2q_native", NATIVE_PATH)
-    mod = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(mod)
+    try:
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+    except ImportError as e:
+        raise RuntimeError(f"{NATIVE_PATH} does not load into {_running()}; run krea-2_amd/build.py") from e
+    # compiled against one torch's C++ classes: another's may lie differently in memory
+    if getattr(mod, "built_for", None) != _running():
+        raise RuntimeError(f"{NATIVE_PATH} was built for {getattr(mod, 'built_for', 'an unknown torch')} and this is "
+                           f"{_running()}; run krea-2_amd/build.py")
     mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _SIGNATURES}, _stream_of_index)
     _native = mod
 

@@ -61,6 +61,8 @@ def _build_native() -> None:
     tmp = NATIVE_LIB.with_suffix(".so.tmp")
     cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           # _lib.py compares this with what runs: the extension is bound to one torch and one Python build
+           f'-DK2Q_BUILT_FOR="torch {torch.__version__}, {sysconfig.get_config_var("SOABI")}"',
            f"-I{sysconfig.get_paths()['include']}", *(f"-isystem{p}" for p in include_paths()), str(BINDING),
            *(f"-L{p}" for p in libs), *(f"-Wl,-rpath,{p}" for p in libs), "-ltorch_python", "-ltorch", "-ltorch_cpu",
            "-lc10", "-o", str(tmp)]

@@ -449,4 +449,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_k2q_native", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__k2q_native() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__k2q_native() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", K2Q_BUILT_FOR) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -61,6 +61,19 @@ def test_failed_allocation_keeps_its_class(k2):
         k2._lib.alloc_codes(x)
 
 
+def test_extension_of_another_torch_is_refused(k2, monkeypatch):
+    L = k2._lib
+    lib = L.load()
+    monkeypatch.setattr(L, "_native", None)
+    monkeypatch.setattr(L.torch, "__version__", "0.0.0")
+    with pytest.raises(RuntimeError, match="run krea-2_amd/build.py"):
+        L._bind_native(lib)
+    assert L._native is None
+    monkeypatch.undo()
+    L._bind_native(lib)
+    assert L._native is not None
+
+
 @pytest.mark.gpu
 def test_out_of_memory_keeps_its_class(k2, dev):
     x = torch.zeros((1, 128), dtype=torch.bfloat16, device=dev).expand(1 << 36, 128)     # codes of 8 TiB
