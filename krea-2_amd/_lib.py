@@ -214,9 +214,10 @@ def _device_check(dev: torch.device) -> None:
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     if idx not in _device_ok:
         with torch.cuda.device(idx):
-            _device_ok[idx] = load().k2q_check_device() == K2Q_OK
-        if _device_ok[idx]:
+            ok = load().k2q_check_device() == K2Q_OK
+        if ok:
             _native.device_checked(idx)
+        _device_ok[idx] = ok     # last: another thread that finds it here goes straight back to the native call
     if not _device_ok[idx]:
         raise RuntimeError(f"device cuda:{idx} is not gfx950 (MI355X); the k2q kernels are built for gfx950 only")
 

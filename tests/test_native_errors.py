@@ -1,6 +1,7 @@
 """Tests of the native wrappers' error paths: an operand without storage (a functorch wrapper) comes back as a Python
 exception, as it does from a ctypes call, whichever operand it is, and an allocation that fails raises what torch.empty
 raises."""
+import contextlib
 import subprocess
 import sys
 from pathlib import Path
@@ -72,6 +73,20 @@ def test_extension_of_another_torch_is_refused(k2, monkeypatch):
     monkeypatch.undo()
     L._bind_native(lib)
     assert L._native is not None
+
+
+def test_device_is_known_to_the_wrappers_before_other_threads_see_it_checked(k2, monkeypatch):
+    """A thread that finds the device checked calls the native wrapper again at once: it must not refuse it then."""
+    L = k2._lib
+    seen = []
+    known = {}
+    monkeypatch.setattr(L, "_device_ok", known)
+    monkeypatch.setattr(L, "load", lambda: type("Lib", (), {"k2q_check_device": staticmethod(lambda: L.K2Q_OK)}))
+    monkeypatch.setattr(L, "_native", type("Native", (), {"device_checked": staticmethod(
+        lambda i: seen.append(dict(known)))}))
+    monkeypatch.setattr(L.torch.cuda, "device", lambda i: contextlib.nullcontext())
+    L._device_check(torch.device("cuda:0"))
+    assert seen == [{}] and known == {0: True}
 
 
 @pytest.mark.gpu
