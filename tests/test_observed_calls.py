@@ -33,6 +33,18 @@ def test_tangents_are_refused(layer):
             layer(forward_ad.make_dual(x, torch.ones_like(x)))
 
 
+@pytest.mark.parametrize("name", ["weight_fp8", "scale", "bias"])
+def test_output_requires_grad_when_a_base_tensor_does(k2, layer, name):
+    """A base unfrozen as a whole: the layer has no gradient for it, and its output still belongs to the graph."""
+    layer.bias = torch.nn.Parameter(torch.zeros(128), requires_grad=False)
+    x = torch.randn(2, 4, 128).to(torch.bfloat16)
+    assert not layer(x).requires_grad
+    getattr(layer, name).requires_grad_()
+    assert layer(x).requires_grad
+    with torch.no_grad():
+        assert not layer(x).requires_grad
+
+
 def test_padding_under_a_tracer_or_a_dual_level_is_torch_operations(k2):
     assert not k2._lib.observed()
     with forward_ad.dual_level():
