@@ -272,7 +272,7 @@ class ConvRotLinear(nn.Module):
         w4 = self.mode == "w4a8"
         grad = torch.is_grad_enabled() and (x2.requires_grad or (lora_A is not None and
                                                                   (lora_A.requires_grad or lora_B.requires_grad)))
-        if grad:
+        if grad or _lib.observed():
             y = _ConvRotLinearFn.apply(x2, lora_A, lora_B, self.qweight, self.weight_scale, self._bias_f32(), w4,
                                        float(lora_scale), qx, sx, ready, self)
         else:   # nothing to differentiate: no autograd node, the one library call (u stays internal)

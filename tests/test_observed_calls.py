@@ -5,17 +5,42 @@ import torch
 from torch.autograd import forward_ad
 
 
-@pytest.fixture
-def layer(k2, monkeypatch):
-    """An fp8 layer whose library calls work on the tensors' values, seen by no tracer and carrying no tangents."""
+def _unseen(t):
+    """The values of ``t`` in a tensor that no tracer and no forward-mode level has seen."""
+    return torch.tensor(t.detach().float().tolist())
+
+
+def _fp8_layer(k2, monkeypatch):
     def forward(x, A, B, q, s, bias, scale):
-        w = torch.tensor(q.float().tolist()) * s.float().view(-1, 1)
-        return torch.tensor((torch.tensor(x.float().tolist()) @ w.t()).tolist(), dtype=torch.bfloat16), None
+        return (_unseen(x) @ (_unseen(q) * _unseen(s).view(-1, 1)).t()).to(torch.bfloat16), None
 
     monkeypatch.setattr(k2.quantize, "_fp8_forward", forward)
-    g = torch.Generator().manual_seed(1)
-    q = torch.randn(128, 128, generator=g).to(torch.float8_e4m3fn)
+    q = torch.randn(128, 128, generator=torch.Generator().manual_seed(1)).to(torch.float8_e4m3fn)
     return k2.Fp8Linear.from_quantized(q, torch.ones(128, dtype=torch.bfloat16), None)
+
+
+def _convrot_layer(k2, monkeypatch):
+    lib = k2.quantize._lib
+
+    def linear_fwd(x2, qx, sx, ready, A, B, scale, qw, sw, bias, w4, need_u=True):
+        return (_unseen(x2) @ _unseen(qw).t()).to(torch.bfloat16), None
+
+    monkeypatch.setattr(lib, "linear_fwd", linear_fwd)
+    monkeypatch.setattr(lib, "alloc_codes", lambda x2: (torch.zeros(x2.shape, dtype=torch.int8), torch.zeros(x2.shape[0])))
+    monkeypatch.setattr(lib, "_stream", lambda dev: 0)
+    q = torch.randint(-9, 10, (128, 128), generator=torch.Generator().manual_seed(1), dtype=torch.int8)
+    return k2.ConvRotLinear.from_quantized(q, torch.zeros(128, dtype=torch.int32), None)
+
+
+@pytest.fixture(params=[_fp8_layer, _convrot_layer])
+def any_layer(k2, monkeypatch, request):
+    """A layer whose library calls work on the tensors' values, as a kernel does."""
+    return request.param(k2, monkeypatch)
+
+
+@pytest.fixture
+def layer(k2, monkeypatch):
+    return _fp8_layer(k2, monkeypatch)
 
 
 def test_trace_follows_its_input(layer):
@@ -25,12 +50,16 @@ def test_trace_follows_its_input(layer):
         assert torch.equal(traced(other), layer(other))
 
 
-def test_tangents_are_refused(layer):
+def test_tangents_are_refused(any_layer):
+    layer = any_layer
     x = torch.randn(4, 128).to(torch.bfloat16)
     with torch.no_grad():
         layer(x)
         with forward_ad.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
             layer(forward_ad.make_dual(x, torch.ones_like(x)))
+        want = layer(x)
+        with forward_ad.dual_level():                # a level without tangents takes the call
+            assert torch.equal(layer(x), want)
 
 
 @pytest.mark.parametrize("name", ["weight_fp8", "scale", "bias"])
