@@ -344,6 +344,13 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// LDS hand-off between the lanes of one wave: the hardware keeps a wave's LDS operations in order, this keeps the
+// compiler from moving a read of what other lanes wrote above the writes.  No instruction.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Workgroup barrier for LDS hand-offs: the wave's own LDS operations complete first (s_barrier alone does
 // not wait for them, and a ds_write still queued when another wave passes the barrier is not yet visible
 // to it); outstanding global loads, the LDS-DMA prefetches among them, are not waited for.
@@ -1180,9 +1187,10 @@ __global__ __launch_bounds__(64 * FIX_WAVES, UMAX > 1 ? 1 : 2) void gemm_fixup_k
         for (int ia = 0; ia < NA; ++ia) f[ia] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ba[ia], bb, f[ia], 0, 0, 0);
       }
     }
-    uint8_t* ct = ctiles[wave];   // this wave's alone: its own LDS operations complete in order
+    uint8_t* ct = ctiles[wave];   // this wave's alone
 #pragma unroll
     for (int ia = 0; ia < NA; ++ia) ctile_put<CROW>(ct, 0, 32 * ia, lane, f[ia]);
+    wave_lds_fence();
     uint16_t* out = static_cast<uint16_t*>(p.out);
     constexpr int CPR = C::ARW / 8, RPI = 64 / CPR;   // 16-byte chunks per row, rows per store instruction
     const int chunk = lane % CPR;
