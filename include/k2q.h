@@ -156,8 +156,17 @@ int k2q_lora_grads_noalloc(const uint16_t* dy, const uint16_t* x, const float* u
  * bias, u, lora_b nullable (r ignored when u is null).  M <= 8 runs a GEMV.  When the 256 x 256 tiles
  * leave the last round of the GPU partly empty, the remainder tiles are cut along K into pieces whose
  * int32 sums meet in ws (k2q_gemm_w8a8_ws_bytes(M, N, K) bytes, 0 = not used); the result is identical.
- * ws == NULL or too small: full-K tiles only. */
+ * ws == NULL or too small: full-K tiles only.
+ * The *_ws_bytes queries of the GEMMs have room for the pieces of any tile shape that a call may be given (the debug
+ * entries below); k2q_gemm_plan_ws_bytes is what the call's own schedule touches, often nothing.  A call with that
+ * much, or with NULL where it is 0, runs the same schedule as with more. */
 int64_t k2q_gemm_w8a8_ws_bytes(int64_t M, int64_t N, int64_t K);
+#define K2Q_GEMM_W8A8 0            /* k2q_gemm_w8a8 */
+#define K2Q_GEMM_W8A8_GROUPED 1    /* k2q_gemm_w8a8_grouped, N the segments' total */
+#define K2Q_GEMM_DX_LIN 2          /* k2q_gemm_dx_lin */
+#define K2Q_GEMM_DX_GROUPED 3      /* k2q_gemm_dx_grouped_ws, N the segments' total */
+#define K2Q_GEMM_BF16 4            /* k2q_gemm_bf16 */
+int64_t k2q_gemm_plan_ws_bytes(int entry, int64_t M, int64_t N, int64_t K);
 int k2q_gemm_w8a8(const int8_t* qx, const float* sx, const int8_t* qw, const float* sw, const float* bias,
                   const float* u, const float* lora_b, int64_t r, float lora_scale,
                   int64_t M, int64_t N, int64_t K, uint16_t* y, void* ws, int64_t ws_bytes, void* stream);
@@ -168,7 +177,8 @@ int k2q_gemm_w8a8(const int8_t* qx, const float* sx, const int8_t* qw, const flo
  * with its factors u[:, u_col .. u_col + r) (u: M rows of ldu f32, r as for k2q_gemm_w8a8; lora_b NULL: no
  * adapter on that segment); the outputs are bit-identical to nseg separate k2q_gemm_w8a8 calls.
  * 1 <= nseg <= 4, every N a multiple of 256, M > 8.  ws: as for k2q_gemm_w8a8 with N the
- * segments' total (k2q_gemm_w8a8_ws_bytes(M, sum_i N_i, K) bytes; NULL: full-K tiles only, the same result). */
+ * segments' total (k2q_gemm_plan_ws_bytes(K2Q_GEMM_W8A8_GROUPED, M, sum_i N_i, K) bytes; NULL: full-K tiles only, the
+ * same result). */
 typedef struct {
   const int8_t* qw;       /* N x K int8 codes */
   const float* sw;        /* N f32 scales */
@@ -197,7 +207,7 @@ int k2q_gemm_w8a8_grouped(const int8_t* qx, const float* sx, int64_t M, int64_t 
  * carries that kernel's summation order).
  * ws: k2q_linear_fwd_ws_bytes bytes (256-byte aligned): factors, their partials and the GEMM's split pieces.
  * It may be NULL when u is given and the call takes u from the rotate/quant pass (k2q_linear_fwd_fuses_down)
- * and, for W8, k2q_gemm_w8a8_ws_bytes(M, N, K) is 0: nothing of it is used then. */
+ * and, for W8, k2q_gemm_plan_ws_bytes(K2Q_GEMM_W8A8, M, N, K) is 0: nothing of it is used then. */
 #define K2Q_WMODE_W8 0
 #define K2Q_WMODE_W4 1
 int64_t k2q_linear_fwd_ws_bytes(int wmode, int64_t M, int64_t N, int64_t K, int64_t r);
@@ -300,8 +310,8 @@ typedef struct {
 int k2q_gemm_dx_grouped(const k2q_dx_segment* seg, int64_t nseg, int64_t M, int64_t K, const float* g, int64_t ldg,
                         const float* lora_a, int64_t r, uint16_t* dx, void* stream);
 /* k2q_gemm_dx_grouped with a workspace for the split schedule (a short last round of tiles over a long reduction is
- * cut along it, as in k2q_gemm_dx_lin; f32 pieces added in a fixed order): k2q_gemm_dx_ws_bytes(M, sum_i N_i, K)
- * bytes.  ws NULL or too small: full-reduction tiles only, what k2q_gemm_dx_grouped runs. */
+ * cut along it, as in k2q_gemm_dx_lin; f32 pieces added in a fixed order):
+ * k2q_gemm_plan_ws_bytes(K2Q_GEMM_DX_GROUPED, M, sum_i N_i, K) bytes.  ws NULL or too small: full-reduction tiles only, what k2q_gemm_dx_grouped runs. */
 int k2q_gemm_dx_grouped_ws(const k2q_dx_segment* seg, int64_t nseg, int64_t M, int64_t K, const float* g, int64_t ldg,
                            const float* lora_a, int64_t r, uint16_t* dx, void* ws, int64_t ws_bytes, void* stream);
 

@@ -79,6 +79,7 @@ _SIGNATURES = {
     "k2q_lora_grads_grouped": ([_p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p, _i64, _p], _int),
     "k2q_lora_grads_noalloc": ([_p, _p, _p, _p, _i64, _f32, _i64, _i64, _i64, _p, _p, _p, _p], _int),
     "k2q_gemm_w8a8_ws_bytes": ([_i64, _i64, _i64], _i64),
+    "k2q_gemm_plan_ws_bytes": ([_int, _i64, _i64, _i64], _i64),
     "k2q_gemm_w8a8": ([_p, _p, _p, _p, _p, _p, _p, _i64, _f32, _i64, _i64, _i64, _p, _p, _i64, _p], _int),
     "k2q_gemm_w8a8_grouped": ([_p, _p, _i64, _i64, _p, _i64, _p, _i64, _i64, _p, _i64, _p], _int),
     "k2q_gemm_w4a8": ([_p, _p, _p, _p, _p, _p, _p, _i64, _f32, _i64, _i64, _i64, _p, _p], _int),
@@ -242,6 +243,14 @@ def _workspace(nbytes: int, dev: torch.device):
     if nbytes <= 0:
         return None, 0
     return torch.empty((nbytes,), dtype=torch.uint8, device=dev), nbytes
+
+
+GEMM_W8A8, GEMM_W8A8_GROUPED, GEMM_DX_LIN, GEMM_DX_GROUPED, GEMM_BF16 = range(5)     # K2Q_GEMM_*
+
+
+def gemm_plan_ws_bytes(entry: int, M: int, N: int, K: int) -> int:
+    """Workspace bytes that a GEMM's own schedule touches (0: its reduction is not cut).  Host only."""
+    return load().k2q_gemm_plan_ws_bytes(entry, M, N, K)
 
 
 def _check_k(K: int) -> None:
@@ -686,7 +695,9 @@ def gemm_w8a8(qx, sx, qw, sw, bias=None, u=None, lora_b=None, lora_scale: float 
     _device_check(dev)
     y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     lib = load()
-    ws, nws = _workspace(lib.k2q_gemm_w8a8_ws_bytes(M, N, K) if split else 0, dev)
+    # a forced shape may cut where the launch's own would not
+    need = gemm_plan_ws_bytes(GEMM_W8A8, M, N, K) if tile == "auto" else lib.k2q_gemm_w8a8_ws_bytes(M, N, K)
+    ws, nws = _workspace(need if split else 0, dev)
     _check(lib.k2q_gemm_w8a8_tile(_ptr(qx), _ptr(sx), _ptr(qw), _ptr(sw), _ptr(bias), _ptr(u), _ptr(lora_b), r,
                                   float(lora_scale), M, N, K, _ptr(y), _ptr(ws), nws, TILES[tile], _stream(dev)),
            "k2q_gemm_w8a8")
@@ -792,7 +803,7 @@ def gemm_w8a8_grouped(qx, sx, segments, u=None):
         arr[i] = W8A8Segment(_ptr(qw), _ptr(sw), _ptr(bias), _ptr(lb), _ptr(y), N, int(u_col or 0), float(scale))
     _device_check(dev)
     lib = load()
-    ws, nws = _workspace(lib.k2q_gemm_w8a8_ws_bytes(M, sum(o.shape[1] for o in outs), K), dev)
+    ws, nws = _workspace(gemm_plan_ws_bytes(GEMM_W8A8_GROUPED, M, sum(o.shape[1] for o in outs), K), dev)
     _check(lib.k2q_gemm_w8a8_grouped(_ptr(qx), _ptr(sx), M, K, ctypes.cast(arr, ctypes.c_void_p), len(segments),
                                      _ptr(u), r, ldu, _ptr(ws), nws, _stream(dev)), "k2q_gemm_w8a8_grouped")
     return outs
@@ -940,7 +951,8 @@ def gemm_dx(dy, qw, sw, *, w4: bool = False, g=None, lora_a=None, split: bool = 
         _check(prep(None if w4 else _ptr(qw), None if w4 else _ptr(sw), _ptr(qw) if w4 else None,
                     _ptr(sw) if w4 else None, N, K, _ptr(wt), st), "k2q_dx_prep")
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
-    ws, nws = _workspace(lib.k2q_gemm_dx_ws_bytes(M, N, K) if split else 0, dev)
+    need = gemm_plan_ws_bytes(GEMM_DX_LIN, M, N, K) if fold_rotation else lib.k2q_gemm_dx_ws_bytes(M, N, K)
+    ws, nws = _workspace(need if split else 0, dev)
     gemm = lib.k2q_gemm_dx_lin if fold_rotation else lib.k2q_gemm_dx
     _check(gemm(_ptr(dy), _ptr(wt), M, N, K, _ptr(g), _ptr(lora_a) if r else None, r, _ptr(dx),
                 _ptr(ws), nws, st), "k2q_gemm_dx")
@@ -986,7 +998,7 @@ def gemm_dx_grouped(segments, g=None, lora_a=None) -> torch.Tensor:
     _device_check(dev)
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
     lib = load()
-    ws, nws = _workspace(lib.k2q_gemm_dx_ws_bytes(M, sum(dy.shape[1] for dy, _ in segments), K), dev)
+    ws, nws = _workspace(gemm_plan_ws_bytes(GEMM_DX_GROUPED, M, sum(dy.shape[1] for dy, _ in segments), K), dev)
     _check(lib.k2q_gemm_dx_grouped_ws(ctypes.addressof(arr), len(segments), M, K, _ptr(g), ldg,
                                       _ptr(lora_a) if r else None, r, _ptr(dx), _ptr(ws), nws, _stream(dev)),
            "k2q_gemm_dx_grouped")
@@ -1068,7 +1080,7 @@ def gemm_bf16(x, w, bias=None, u=None, lora_b=None, lora_scale: float = 1.0, *, 
     _device_check(dev)
     lib = load()
     y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-    ws, nws = _workspace(lib.k2q_gemm_bf16_ws_bytes(M, N, K) if split else 0, dev)
+    ws, nws = _workspace(gemm_plan_ws_bytes(GEMM_BF16, M, N, K) if split else 0, dev)
     _check(lib.k2q_gemm_bf16(_ptr(x), _ptr(w), _ptr(bias), _ptr(u), _ptr(lora_b), r, float(lora_scale), M, N, K,
                              _ptr(y), _ptr(ws), nws, _stream(dev)), "k2q_gemm_bf16")
     return y
@@ -1101,7 +1113,7 @@ def gemm_dx_fp8(dy, q, s, *, g=None, lora_a=None, split: bool = True) -> torch.T
         if dx.__class__ is int:
             _check(dx, "k2q_gemm_dx_lin")
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
-    ws, nws = _workspace(lib.k2q_gemm_dx_ws_bytes(M, N, K) if split else 0, dev)
+    ws, nws = _workspace(gemm_plan_ws_bytes(GEMM_DX_LIN, M, N, K) if split else 0, dev)
     _check(lib.k2q_gemm_dx_lin(_ptr(dy), _ptr(wt), M, N, K, _ptr(g), _ptr(lora_a) if r else None, r, _ptr(dx),
                                _ptr(ws), nws, st), "k2q_gemm_dx_lin")
     return dx

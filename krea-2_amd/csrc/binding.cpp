@@ -30,10 +30,9 @@ struct Api {
   decltype(&k2q_pad_factors) pad_factors;
   decltype(&k2q_dx_prep_eff) dx_prep_eff;
   decltype(&k2q_gemm_dx_lin) gemm_dx_lin;
-  decltype(&k2q_gemm_dx_ws_bytes) gemm_dx_ws_bytes;
   decltype(&k2q_dequant_fp8) dequant_fp8;
   decltype(&k2q_gemm_bf16) gemm_bf16;
-  decltype(&k2q_gemm_bf16_ws_bytes) gemm_bf16_ws_bytes;
+  decltype(&k2q_gemm_plan_ws_bytes) gemm_plan_ws_bytes;
 } api{};
 
 PyObject* raw_stream_of = nullptr;   // torch._C._cuda_getCurrentRawStream
@@ -309,7 +308,7 @@ PyObject* dx_lin(const Tensor& dy, const Tensor& wt, const Tensor* g, const Tens
   const int64_t M = dy.size(0), N = dy.size(1), K = wt.size(0), r = g ? g->size(1) : 0;
   const c10::Device d = dy.device();
   Tensor dx = alloc({M, K}, at::kBFloat16, d);
-  const int64_t nws = api.gemm_dx_ws_bytes(M, N, K);
+  const int64_t nws = api.gemm_plan_ws_bytes(K2Q_GEMM_DX_LIN, M, N, K);
   Tensor ws = workspace(nws, d);
   const int rc = foreign(api.gemm_dx_lin, as<uint16_t>(dy.data_ptr()), as<uint16_t>(wt.data_ptr()), M, N, K,
                          as<float>(ptr(g)), r ? as<float>(ptr(A)) : nullptr, r, as<uint16_t>(dx.data_ptr()), ptr(ws),
@@ -394,7 +393,7 @@ PyObject* py_gemm_bf16(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* st;
     if (!stream_of(d, st)) return nullptr;
     Tensor y = alloc({M, N}, at::kBFloat16, d);
-    const int64_t nws = api.gemm_bf16_ws_bytes(M, N, K);
+    const int64_t nws = api.gemm_plan_ws_bytes(K2Q_GEMM_BF16, M, N, K);
     Tensor ws = workspace(nws, d);
     const int rc = foreign(api.gemm_bf16, as<uint16_t>(ptr(x)), as<uint16_t>(ptr(w)), as<float>(ptr(bias)),
                            as<float>(ptr(u)), u ? as<float>(ptr(B)) : nullptr, r, (float)scale, M, N, K,
@@ -420,10 +419,9 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
       !get("k2q_linear_fwd_fuses_down", api.linear_fwd_fuses_down) || !get("k2q_lora_grads", api.lora_grads) ||
       !get("k2q_lora_grads_ws_bytes", api.lora_grads_ws_bytes) || !get("k2q_lora_down", api.lora_down) ||
       !get("k2q_lora_down_ws_bytes", api.lora_down_ws_bytes) || !get("k2q_pad_factors", api.pad_factors) ||
-      !get("k2q_dx_prep_eff", api.dx_prep_eff) ||
-      !get("k2q_gemm_dx_lin", api.gemm_dx_lin) || !get("k2q_gemm_dx_ws_bytes", api.gemm_dx_ws_bytes) ||
+      !get("k2q_dx_prep_eff", api.dx_prep_eff) || !get("k2q_gemm_dx_lin", api.gemm_dx_lin) ||
       !get("k2q_dequant_fp8", api.dequant_fp8) || !get("k2q_gemm_bf16", api.gemm_bf16) ||
-      !get("k2q_gemm_bf16_ws_bytes", api.gemm_bf16_ws_bytes))
+      !get("k2q_gemm_plan_ws_bytes", api.gemm_plan_ws_bytes))
     return nullptr;
   Py_INCREF(a[1]);
   Py_XSETREF(raw_stream_of, a[1]);

@@ -1698,17 +1698,28 @@ unsigned allowed_tiles(bool grouped, bool ksegs) {
   return m;
 }
 
-// Workspace for any schedule an entry may take: the larger of the T256 and T128 plans' pieces (used when the launch
-// runs that tile shape, chosen or forced; other shapes leave it untouched).
+// Whether a launch may cut its last round, given room for the pieces.
+bool may_split(bool ksegs, int64_t kbytes) { return !ksegs || kbytes / WBK >= KSEG_SPLIT_MIN; }
+
+int64_t piece_bytes(const TileChoice& c) {
+  return c.split.s > 1 ? (int64_t)c.split.rem * c.split.s * TILE_COSTS[c.tile].ta * TILE_COSTS[c.tile].tb * 4 : 0;
+}
+
+// Workspace that holds the pieces of the T256 plan and of the T128 plan, whichever shape a launch is given.
 int64_t split_ws_bytes(bool bf16, int64_t rows_a, int64_t rows_b, int64_t kbytes) {
   const int cus = k2q_cu_count();
   int64_t bytes = 0;
   for (int t : {TILE_256, TILE_128}) {
-    const SplitPlan q = tile_plan(t, bf16, rows_a, rows_b, (int)(kbytes / WBK), cus, true);
-    const int64_t b = q.s > 1 ? (int64_t)q.rem * q.s * TILE_COSTS[t].ta * TILE_COSTS[t].tb * 4 : 0;
+    const int64_t b = piece_bytes({t, tile_plan(t, bf16, rows_a, rows_b, (int)(kbytes / WBK), cus, true)});
     bytes = b > bytes ? b : bytes;
   }
   return bytes;
+}
+
+// Workspace of the schedule that a launch takes when it has one.
+int64_t plan_ws_bytes(int epi, int64_t rows_a, int64_t rows_b, int64_t kbytes, bool grouped, bool ksegs) {
+  return piece_bytes(choose_tile(epi, rows_a, rows_b, kbytes, allowed_tiles(grouped, ksegs), may_split(ksegs, kbytes),
+                                 TILE_AUTO, k2q_cu_count()));
 }
 
 template <int EPI, int MODE, class C, int NS>
@@ -1845,9 +1856,12 @@ int launch_gemm(GemmArgs p, void* ws, int64_t ws_bytes, hipStream_t st, int forc
   }
   if (320 * ld_max >= 0x7fffffffLL) return K2Q_EUNSUPPORTED;
   if (forced >= TILE_COUNT || (EPI == EPI_DX && forced >= 0 && forced != TILE_256)) return K2Q_EINVAL;
-  TileChoice c = choose_tile(EPI, p.rows_a, p.rows_b, p.kbytes, allowed_tiles(p.nseg > 0, p.nks > 0),
-                             ws != nullptr && (p.nks == 0 || p.kbytes / WBK >= KSEG_SPLIT_MIN), forced,
-                             k2q_cu_count());
+  auto choose = [&](bool split) {
+    return choose_tile(EPI, p.rows_a, p.rows_b, p.kbytes, allowed_tiles(p.nseg > 0, p.nks > 0), split, forced,
+                       k2q_cu_count());
+  };
+  TileChoice c = choose(ws != nullptr && k2q_aligned(ws, 16) && may_split(p.nks > 0, p.kbytes));
+  if (ws_bytes < piece_bytes(c)) c = choose(false);   // no room for the pieces: what a launch without ws runs
   if (forced >= 0 && !(allowed_tiles(p.nseg > 0, p.nks > 0) >> forced & 1)) return K2Q_EINVAL;
   if (p.nseg > 0) {   // segments start on tile boundaries
     const int ta = c.tile == TILE_192 ? 192 : c.tile == TILE_128 ? 128 : 256;
@@ -1863,10 +1877,7 @@ int launch_gemm(GemmArgs p, void* ws, int64_t ws_bytes, hipStream_t st, int forc
     p.dp_tiles = tiles;
     p.sk_rem = 0;
     p.sk_s = 1;
-    SplitPlan q = c.split;
-    if (c.tile != TILE_128 || (q.s > 1 && (!ws || ws_bytes < (int64_t)q.rem * q.s * 128 * 128 * 4 ||
-                                           !k2q_aligned(ws, 16))))
-      q = SplitPlan{tiles, 0, 1, 0.0};   // no split, or no room for the pieces: full-K tiles only
+    const SplitPlan q = c.split;   // s > 1: T128
     {
       const int tar = c.tile == TILE_320 ? 256 : c.tile == TILE_192 ? 192 : 128;
       const int tbr = c.tile == TILE_320 ? 320 : c.tile == TILE_192 ? 256 : 128;
@@ -1895,11 +1906,9 @@ int launch_gemm(GemmArgs p, void* ws, int64_t ws_bytes, hipStream_t st, int forc
     }
     return rc ? rc : k2q_launch_status();
   }
-  SplitPlan q = c.split;
+  const SplitPlan q = c.split;
   const int64_t tiles = ((p.rows_a + 255) / 256) * ((p.rows_b + 255) / 256);
   if (tiles > 0x7fffffff) return K2Q_EUNSUPPORTED;
-  if (q.s > 1 && (!ws || ws_bytes < (int64_t)q.rem * q.s * 256 * 256 * 4 || !k2q_aligned(ws, 16)))
-    q = SplitPlan{tiles, 0, 1, 0.0};   // no room for the pieces: full-K tiles only
   p.dp_tiles = q.dp_tiles;
   p.sk_rem = q.rem;
   p.sk_s = q.s;
@@ -1936,6 +1945,23 @@ extern "C" int64_t k2q_gemm_w8a8_ws_bytes(int64_t M, int64_t N, int64_t K) {
 extern "C" int64_t k2q_gemm_dx_ws_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || K < K2Q_HADAMARD || K % K2Q_HADAMARD || N < 64 || N % 64) return 0;
   return split_ws_bytes(true, K, M, 2 * N);
+}
+
+extern "C" int64_t k2q_gemm_plan_ws_bytes(int entry, int64_t M, int64_t N, int64_t K) {
+  switch (entry) {
+    case K2Q_GEMM_W8A8:
+    case K2Q_GEMM_W8A8_GROUPED:
+      if (check_common(M, N, K) || M <= K2Q_GEMV_MAX_M) return 0;
+      return plan_ws_bytes(EPI_W8, N, M, K, entry == K2Q_GEMM_W8A8_GROUPED, false);
+    case K2Q_GEMM_DX_LIN:
+    case K2Q_GEMM_DX_GROUPED:
+      if (M < 1 || K < K2Q_HADAMARD || K % K2Q_HADAMARD || N < 64 || N % 64) return 0;
+      return plan_ws_bytes(EPI_DXLIN, K, M, 2 * N, false, entry == K2Q_GEMM_DX_GROUPED);
+    case K2Q_GEMM_BF16:
+      if (M < 1 || N < 1 || N % 4 || K < 64 || K % 64) return 0;
+      return plan_ws_bytes(EPI_LIN, N, M, 2 * K, false, false);
+    default: return 0;
+  }
 }
 
 extern "C" int k2q_gemm_w8a8(const int8_t* qx, const float* sx, const int8_t* qw, const float* sw,

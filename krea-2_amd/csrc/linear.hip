@@ -142,7 +142,7 @@ FwdLayout fwd_layout(int wmode, int64_t M, int64_t N, int64_t K, int64_t r) {
     off += align256(a > b ? a : b);
   }
   L.gemm_off = off;
-  off += align256(wmode == K2Q_WMODE_W8 ? k2q_gemm_w8a8_ws_bytes(M, N, K) : gemm_w4a8_ws_bytes(M, N, K));
+  off += align256(wmode == K2Q_WMODE_W8 ? k2q_gemm_plan_ws_bytes(K2Q_GEMM_W8A8, M, N, K) : gemm_w4a8_ws_bytes(M, N, K));
   L.total = off;
   return L;
 }
