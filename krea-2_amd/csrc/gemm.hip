@@ -1575,16 +1575,18 @@ template <int EPI, class C>
 int launch_w4_tile(W4Args p, hipStream_t st) {
   const int64_t tiles = w4_tiles(p.M, p.N, C::IB);
   if (tiles > 0x7fffffff) return K2Q_EUNSUPPORTED;
-  if (p.s > 1) {
-    static std::atomic<uint64_t> set_p{0};
-    if (k2q_lds_limit_once(gemm_w4_kernel<EPI, C, true>, C::LDS, set_p)) return K2Q_ELAUNCH;
-    hipLaunchKernelGGL((gemm_w4_kernel<EPI, C, true>), dim3((unsigned)tiles, (unsigned)p.s), dim3(256), C::LDS, st, p);
-    hipLaunchKernelGGL((w4_fixup_kernel<EPI, C>), dim3((unsigned)tiles, C::IB), dim3(256), 0, st, p);
-  } else {
-    static std::atomic<uint64_t> set_t{0};
-    if (k2q_lds_limit_once(gemm_w4_kernel<EPI, C, false>, C::LDS, set_t)) return K2Q_ELAUNCH;
-    hipLaunchKernelGGL((gemm_w4_kernel<EPI, C, false>), dim3((unsigned)tiles), dim3(256), C::LDS, st, p);
+  if constexpr (EPI == EPI_W8) {   // the debug entry has no workspace for pieces
+    if (p.s > 1) {
+      static std::atomic<uint64_t> set_p{0};
+      if (k2q_lds_limit_once(gemm_w4_kernel<EPI, C, true>, C::LDS, set_p)) return K2Q_ELAUNCH;
+      hipLaunchKernelGGL((gemm_w4_kernel<EPI, C, true>), dim3((unsigned)tiles, (unsigned)p.s), dim3(256), C::LDS, st, p);
+      hipLaunchKernelGGL((w4_fixup_kernel<EPI, C>), dim3((unsigned)tiles, C::IB), dim3(256), 0, st, p);
+      return k2q_launch_status();
+    }
   }
+  static std::atomic<uint64_t> set_t{0};
+  if (k2q_lds_limit_once(gemm_w4_kernel<EPI, C, false>, C::LDS, set_t)) return K2Q_ELAUNCH;
+  hipLaunchKernelGGL((gemm_w4_kernel<EPI, C, false>), dim3((unsigned)tiles), dim3(256), C::LDS, st, p);
   return k2q_launch_status();
 }
 
