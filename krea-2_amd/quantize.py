@@ -446,12 +446,14 @@ class Fp8Linear(nn.Module):
         # the reference adds the bias in x.dtype (quantize.py:50): round it to bf16 first
         b = self.bias.to(torch.bfloat16).float().contiguous() if self.bias is not None else None
         scale = self.scale.to(torch.bfloat16).contiguous()
-        grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x2, lora_A, lora_B,
-                                                                                           self.weight_fp8, scale, b))
+        q = self.weight_fp8
+        grad = torch.is_grad_enabled() and (
+            x2.requires_grad or q.requires_grad or scale.requires_grad or (b is not None and b.requires_grad)
+            or (lora_A is not None and (lora_A.requires_grad or lora_B.requires_grad)))
         if grad or _lib.observed():
-            y = _Fp8LinearFn.apply(x2, lora_A, lora_B, self.weight_fp8, scale, b, float(lora_scale))
+            y = _Fp8LinearFn.apply(x2, lora_A, lora_B, q, scale, b, float(lora_scale))
         else:   # no input that requires a gradient: no autograd node
-            y, _ = _fp8_forward(x2, lora_A, lora_B, self.weight_fp8, scale, b, float(lora_scale))
+            y, _ = _fp8_forward(x2, lora_A, lora_B, q, scale, b, float(lora_scale))
         return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.out_features)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
