@@ -90,6 +90,7 @@ _SIGNATURES = {
     "k2q_gemm_w8a8_acc": ([_p, _p, _i64, _i64, _i64, _p, _p, _i64, _int, _p], _int),
     "k2q_gemm_w8a8_tile": ([_p, _p, _p, _p, _p, _p, _p, _i64, _f32, _i64, _i64, _i64, _p, _p, _i64, _int, _p], _int),
     "k2q_gemm_w8a8_plan": ([_i64, _i64, _i64, _int, _int, ctypes.POINTER(_int)], _int),
+    "k2q_gemm_w4a8_plan": ([_i64, _i64, _i64, _int, _int, _p], _int),
     "k2q_gemm_w4a8_f32": ([_p, _p, _p, _i64, _i64, _i64, _p, _p], _int),
     "k2q_quant_weight_fp8": ([_p, _int, _i64, _i64, _p, _p, _p], _int),
     "k2q_dequant_fp8": ([_p, _p, _i64, _i64, _int, _p, _p], _int),
@@ -676,6 +677,16 @@ def gemm_w8a8_plan(M: int, N: int, K: int, cus: int = 256, grouped: bool = False
     if rc < 0:
         _check(rc, "k2q_gemm_w8a8_plan")
     return _TILE_NAMES[rc], pieces.value
+
+
+def gemm_w4a8_plan(M: int, N: int, K: int, cus: int = 256, workspace: bool = True) -> tuple[int, int]:
+    """The schedule of the W4A8 GEMM: (rows per tile, K-pieces per tile) of :func:`linear_fwd` (``workspace``) or of
+    :func:`gemm_w4a8`, which has no room for pieces.  Host only."""
+    pieces = _int(0)
+    rc = load().k2q_gemm_w4a8_plan(M, N, K, cus, int(workspace), ctypes.byref(pieces))
+    if rc < 0:
+        _check(rc, "k2q_gemm_w4a8_plan")
+    return rc, pieces.value
 
 
 def gemm_w8a8(qx, sx, qw, sw, bias=None, u=None, lora_b=None, lora_scale: float = 1.0, *,

@@ -2170,6 +2170,13 @@ int64_t gemm_w4a8_ws_bytes(int64_t M, int64_t N, int64_t K) {
   return w4_piece_bytes(M, N, w4_plan(M, N, K, k2q_cu_count(), true));
 }
 
+extern "C" int k2q_gemm_w4a8_plan(int64_t M, int64_t N, int64_t K, int cus, int workspace, int* split_pieces) {
+  if (check_common(M, N, K) || cus < 1) return K2Q_EINVAL;
+  const W4Plan q = w4_plan(M, N, K, cus, workspace != 0);
+  if (split_pieces) *split_pieces = q.s;
+  return 32 * q.ib;
+}
+
 extern "C" int k2q_gemm_w4a8(const int8_t* qx, const float* sx, const uint8_t* qw4, const uint16_t* sw4,
                              const float* bias, const float* u, const float* lora_b, int64_t r,
                              float lora_scale, int64_t M, int64_t N, int64_t K, uint16_t* y, void* stream) {

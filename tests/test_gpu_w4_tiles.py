@@ -1,8 +1,8 @@
-"""GPU tests of the W4A8 GEMM's tile heights and K-pieces.
+"""GPU tests of the W4A8 GEMM's tile heights and K-pieces; the plan says which of them a shape runs.
 
 With power-of-two group scales and small codes every partial sum is a multiple of one power of two below 2^24 of them, so
-any order of the f32 sums is exact: the one-call forward (which may cut the reduction) must equal the debug entry's
-sums put through the epilogue in float64 and rounded once.  With drawn scales the two schedules agree to f32 rounding.
+any order of the f32 sums is exact: the one-call forward (which may cut the reduction) must equal the product in float64
+rounded once, with whole-number biases and LoRA factors too.  With drawn scales the two schedules agree to f32 rounding.
 """
 import pytest
 import torch
@@ -53,6 +53,8 @@ def test_forward_equals_exact_product(k2, dev, M, N, K, r):
 @pytest.mark.parametrize("M,N,K", [(2, 3072, 12288), (77, 6144, 6144), (333, 3072, 12288), (768, 6144, 16384)])
 def test_pieces_agree_with_full_reduction(k2, dev, M, N, K):
     L = k2._lib
+    assert L.gemm_w4a8_plan(M, N, K)[1] > 1                          # cut with a workspace, whole without
+    assert L.gemm_w4a8_plan(M, N, K, workspace=False)[1] == 1
     g = torch.Generator(device=dev).manual_seed(M + K)
     qx = torch.randint(-127, 128, (M, K), device=dev, dtype=torch.int8, generator=g)
     q4 = torch.randint(0, 256, (N, K // 2), device=dev, dtype=torch.uint8, generator=g)
@@ -67,3 +69,35 @@ def test_pieces_agree_with_full_reduction(k2, dev, M, N, K):
     e = lambda t: ((t.double() - ref).norm() / ref.norm()).item()    # noqa: E731
     full = L.gemm_w4a8(qx, sx, q4, s4)                               # no workspace: the full reduction per tile
     assert e(y) < 2 ** -8 and e(y) < 1.02 * e(full)
+
+
+# (M, N, K, r, rows per tile, pieces): each height cut and whole, ragged last tiles in both directions
+HEIGHTS = [(8, 18432, 3072, 16, 32, 3), (129, 1536, 6144, 48, 32, 8), (333, 3072, 3072, 48, 32, 1),
+           (33, 3072, 3072, 48, 64, 8), (257, 6144, 6144, 16, 64, 3), (4096, 516, 6144, 48, 64, 3),
+           (2100, 3072, 640, 16, 64, 1), (512, 6144, 12288, 16, 128, 4), (1025, 3072, 12288, 48, 128, 3),
+           (4096, 260, 16384, 32, 128, 8), (1025, 18432, 1024, 48, 128, 1)]
+
+
+@pytest.mark.parametrize("M,N,K,r,rows,pieces", HEIGHTS)
+def test_bias_and_factors_in_every_height(k2, dev, M, N, K, r, rows, pieces):
+    L = k2._lib
+    assert L.gemm_w4a8_plan(M, N, K) == (rows, pieces)
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    qx = torch.randint(-127, 128, (M, K), device=dev, dtype=torch.int8, generator=g)
+    q4 = torch.randint(0, 256, (N, K // 2), device=dev, dtype=torch.uint8, generator=g)
+    s4 = torch.exp2(torch.randint(-1, 1, (K // 64, N), device=dev, generator=g).float()).bfloat16()
+    sx = torch.ones(M, device=dev)
+    bias = torch.randint(-40, 41, (N,), device=dev, generator=g).float()
+    x = torch.zeros(M, K, device=dev)                                # |u| <= 16 * 3 * 2: exact in bf16
+    x[:, :16] = torch.randint(-3, 4, (M, 16), device=dev, generator=g).float()
+    A = torch.randint(-2, 3, (r, K), device=dev, generator=g).float()
+    B = torch.randint(-3, 4, (N, r), device=dev, generator=g).float()
+    w = (_codes(q4).double().view(N, -1, 64) * s4.t().double().unsqueeze(-1)).view(N, K)
+    acc = qx.double() @ w.t()
+    u = x.double() @ A.double().t()
+    full = acc / 128 + bias.double() + 2.0 * (u @ B.double().t())
+    assert acc.abs().max() * 2 < 2 ** 24 and full.abs().max() * 2 ** 8 < 2 ** 24       # every f32 sum is exact
+    for need_u in (True, False):
+        y, got = L.linear_fwd(x.bfloat16(), qx, sx, True, A, B, 2.0, q4, s4, bias, True, need_u=need_u)
+        assert torch.equal(y, full.bfloat16())
+        assert not need_u or torch.equal(got.double(), u)

@@ -42,3 +42,18 @@ def test_cut_launches_ask_for_their_pieces(k2, entry, M, N, K):
     L = k2._lib
     assert L.gemm_plan_ws_bytes(getattr(L, entry), M, N, K) >= 2 * 128 * 128 * 4
     assert L.gemm_plan_ws_bytes(getattr(L, entry), M, N + 4, K + 4) == 0        # widths that no kernel takes
+
+
+def test_w4_plan_reports_heights_and_pieces(k2):
+    L = k2._lib
+    assert L.gemm_w4a8_plan(333, 3072, 3072) == (32, 1)
+    assert L.gemm_w4a8_plan(257, 6144, 6144) == (64, 3)
+    assert L.gemm_w4a8_plan(512, 6144, 12288) == (128, 4)
+    assert L.gemm_w4a8_plan(4096, 3072, 3072) == (128, 1)
+    assert L.gemm_w4a8_plan(512, 6144, 12288, workspace=False)[1] == 1
+    for M, N, K in SHAPES:
+        rows, pieces = L.gemm_w4a8_plan(M, N, K)
+        need = -(-N // 128) * -(-M // rows) * pieces * 128 * rows * 4 if pieces > 1 else 0
+        assert L.load().k2q_linear_fwd_ws_bytes(1, M, N, K, 0) == -(-need // 256) * 256
+    with pytest.raises(RuntimeError):
+        L.gemm_w4a8_plan(8, 3072, 100)
