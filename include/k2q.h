@@ -153,8 +153,8 @@ int k2q_lora_grads_noalloc(const uint16_t* dy, const uint16_t* x, const float* u
 /* (2)+(3) W8A8 GEMM with the fused epilogue, replacing F.linear(x, W_deq, b) of quantize.py:49-51 and
  * the LoRA add of lora.py:47-48:
  *   y = bf16(2^-7 s_x[m] s_w[n] acc[m,n] + bias[n] + lora_scale * sum_j u[m,j] lora_b[n,j]).
- * bias, u, lora_b nullable (r ignored when u is null).  M <= 8 runs a GEMV.  When the 256 x 256 tiles
- * leave the last round of the GPU partly empty, the remainder tiles are cut along K into pieces whose
+ * bias, u, lora_b nullable (r ignored when u is null).  M <= 8 runs a GEMV.  When 256 x 256 or 128 x 128 tiles
+ * leave the last round of the GPU partly empty, its tiles may be cut along K into pieces whose
  * int32 sums meet in ws (k2q_gemm_w8a8_ws_bytes(M, N, K) bytes, 0 = not used); the result is identical.
  * ws == NULL or too small: full-K tiles only.
  * The *_ws_bytes queries of the GEMMs have room for the pieces of any tile shape that a call may be given (the debug
@@ -206,8 +206,12 @@ int k2q_gemm_w8a8_grouped(const int8_t* qx, const float* sx, int64_t M, int64_t 
  * tiles), the codes and u come from one k2q_rotquant_lora launch instead of k2q_rotquant + k2q_lora_down (u then
  * carries that kernel's summation order).
  * ws: k2q_linear_fwd_ws_bytes bytes (256-byte aligned): factors, their partials and the GEMM's split pieces.
- * It may be NULL when u is given and the call takes u from the rotate/quant pass (k2q_linear_fwd_fuses_down)
- * and, for W8, k2q_gemm_plan_ws_bytes(K2Q_GEMM_W8A8, M, N, K) is 0: nothing of it is used then. */
+ * It may be NULL when u is given and the call takes u from the rotate/quant pass (k2q_linear_fwd_fuses_down): for W8
+ * with k2q_gemm_plan_ws_bytes(K2Q_GEMM_W8A8, M, N, K) 0 nothing of it is used then, and otherwise the GEMM runs
+ * without cutting its reduction.
+ * The W8 output is the same either way (int32 sums).  W4 adds f32 group sums: its tiles may be cut along K and their
+ * pieces added in a fixed order (k2q_gemm_w4a8_plan), so calls whose plans differ (another M, NULL or a short ws, the
+ * separate k2q_gemm_w4a8) agree to f32 rounding of those sums, and equal calls bit for bit. */
 #define K2Q_WMODE_W8 0
 #define K2Q_WMODE_W4 1
 int64_t k2q_linear_fwd_ws_bytes(int wmode, int64_t M, int64_t N, int64_t K, int64_t r);
@@ -219,14 +223,14 @@ int k2q_linear_fwd(const uint16_t* x, int64_t ldx, int64_t M, int64_t K, int8_t*
                    const void* qw, const void* sw, const float* bias, int64_t N, uint16_t* y, void* ws,
                    int64_t ws_bytes, void* stream);
 
-/* W4A8 variant: per-group int32 partials scaled by the bf16 group scales. */
+/* W4A8 variant: per-group int32 partials scaled by the bf16 group scales and added in f32 over the whole K. */
 int k2q_gemm_w4a8(const int8_t* qx, const float* sx, const uint8_t* qw4, const uint16_t* sw4,
                   const float* bias, const float* u, const float* lora_b, int64_t r, float lora_scale,
                   int64_t M, int64_t N, int64_t K, uint16_t* y, void* stream);
 
 /* Output tile shapes of the MFMA GEMMs (A-rows x B-rows per workgroup).  Every entry point picks one per
  * launch with a cost model (K2Q_TILE_AUTO); the debug entries below take a shape explicitly so tests can run
- * each on any problem.  The result does not depend on the shape (int32 sums are exact; the f32 epilogue and
+ * each on any problem.  The W8 result does not depend on the shape (int32 sums are exact; the f32 epilogue and
  * the LoRA term are computed per element in the same order). */
 #define K2Q_TILE_AUTO (-1)
 #define K2Q_TILE_256x256 0
@@ -237,7 +241,7 @@ int k2q_gemm_w4a8(const int8_t* qx, const float* sx, const uint8_t* qw4, const u
 
 /* The schedule k2q_gemm_w8a8 (and the W8 GEMM of k2q_linear_fwd) takes for an M x N x K problem on a GPU with
  * `cus` compute units: returns the K2Q_TILE_* shape (or K2Q_TILE_GEMV), and in *split_pieces (nullable) the
- * number of K-pieces its last round of 256x256 tiles is cut into (1 = none).  grouped != 0: the schedule of
+ * number of K-pieces its last round of 256x256 or 128x128 tiles is cut into (1 = none).  grouped != 0: the schedule of
  * k2q_gemm_w8a8_grouped with N the segments' total out_features.  Host only: no device call. */
 int k2q_gemm_w8a8_plan(int64_t M, int64_t N, int64_t K, int cus, int grouped, int* split_pieces);
 /* The same for W4: returns the rows per tile (32, 64 or 128) and the K-pieces that every tile is cut into (1 = none).

@@ -671,7 +671,7 @@ _TILE_NAMES = {v: k for k, v in TILES.items()} | {4: "gemv"}
 def gemm_w8a8_plan(M: int, N: int, K: int, cus: int = 256, grouped: bool = False) -> tuple[str, int]:
     """The schedule ``k2q_gemm_w8a8`` (``grouped``: ``k2q_gemm_w8a8_grouped``, N = the segments' total) takes for
     an M x N x K problem on a GPU with ``cus`` compute units: (tile shape or "gemv", K-pieces of the last round
-    of 256x256 tiles).  Host only."""
+    of 256x256 or 128x128 tiles).  Host only."""
     pieces = _int(0)
     rc = load().k2q_gemm_w8a8_plan(M, N, K, cus, int(grouped), ctypes.byref(pieces))
     if rc < 0:

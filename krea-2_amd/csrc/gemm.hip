@@ -141,7 +141,7 @@ __device__ __forceinline__ void group_coords32(uint32_t lid, uint32_t tiles_a, u
   ta = r / gsize;
 }
 
-// For the W4 kernel, whose grid is one workgroup per tile.
+// For the W4 kernel, whose grid is one workgroup per tile in x (and piece in y).
 __device__ __forceinline__ void tile_coords(uint32_t tiles_a, uint32_t tiles_b, uint32_t& ta, uint32_t& tb) {
   group_coords32((uint32_t)xcd_remap(blockIdx.x, tiles_a * tiles_b), tiles_a, tiles_b, 8, ta, tb);
 }
@@ -476,7 +476,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgsN<NS>& p0, int64_t lid, 
     rsa = k2q_rsrc(a + A0 * lda + kb, na * lda - kb);
     rsb = k2q_rsrc(b + B0 * ldb + kb, nb * ldb - kb);
   };
-  // Segmented reduction (full-K tiles of EPI_DXLIN only): stage st of segment j reads its operands at stage
+  // Segmented reduction (EPI_DXLIN, full-K tiles and pieces): stage st of segment j reads its operands at stage
   // st - kbase; seek(st) moves to st's segment.  The stages passed to seek increase by at most one per call
   // and every segment holds at least one stage, so one step per call reaches it.
   // A piece's stages count from its first one, s0 of the whole reduction: the segment tables are moved by s0.

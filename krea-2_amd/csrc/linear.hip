@@ -207,7 +207,8 @@ extern "C" int k2q_linear_fwd(const uint16_t* x, int64_t ldx, int64_t M, int64_t
   if (ws && !k2q_aligned(ws, 256)) return K2Q_EINVAL;
   if (skinny && lora_a && !u) return K2Q_EINVAL;      // the prologue writes u
   uint8_t* w = static_cast<uint8_t*>(ws);
-  // the GEMM's split pieces (without room for them it runs full-K tiles: the same output)
+  // the GEMM's split pieces (without room for them it runs full-K tiles: the same output for W8, for W4 its f32 group
+  // sums in another order)
   void* gws = ws && ws_bytes > lay.gemm_off ? static_cast<void*>(w + lay.gemm_off) : nullptr;
   const int64_t gws_bytes = gws ? ws_bytes - lay.gemm_off : 0;
   int rc = K2Q_OK;
