@@ -102,7 +102,7 @@ struct Raw8<float> {
 // The row-resident quantizer: WPR waves own a row, each lane holds 8 elements of every chunk of 512 WPR in
 // registers, so a weight is read once.  Bound by HBM (2 or 4 bytes in, 1 out per weight); the general kernel above
 // is bound by its 2-byte loads and a full division sequence per element.  16384 x 6144 bf16 (302 MB), a pass among
-// others: 176.3 -> 54.9 us (1.7 -> 5.5 TB/s; a large copy reaches 5.0 TB/s on the same box).
+// others: 176.3 -> 54.6 us (1.7 -> 5.5 TB/s; a large copy reaches 4.7-5.4 TB/s, two reads to a write 6.0).
 //
 // The quotient v / scale is the correctly rounded one, as torch's division gives it (bf16 weights make exact
 // ties between two codes common): with y = RN(1 / scale), q0 = v y is within two units in the last place; one

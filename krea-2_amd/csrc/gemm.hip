@@ -1533,12 +1533,13 @@ int64_t w4_piece_bytes(int64_t M, int64_t N, const W4Plan& q) {
 
 // The cheapest of the heights and 1-8 pieces, estimated in microseconds: a stage of a CU that runs w workgroups costs
 // a + b w (latency, then the scaling's VALU work), a round of CUs x workgroups-per-CU its stages + e, pieces 4.2 +
-// 0.262 per MB.  A partly filled round is priced between its fullest CUs and the average one.  Fitted to the measured
-// times of every height and split at 119 launches (M 1-8192, N 1024-18432, K 1024-16384): 1.5 % from the fastest
-// measured plan on average.  Against the 128-row tiles over the full reduction that every launch took before:
-// 1 x 3072 x 12288 108.5 -> 16.4 us, 333 x 3072 x 3072 30.3 -> 17.2, 768 x 6144 x 6144 69.6 -> 54.0, 1024 x 12288 ->
-// 3072 107.9 -> 65.9; from 2048 rows the 128-row tiles are the faster ones again (4096 x 3072 x 3072 55.1 against
-// 61.6 and 76.4 for 64 and 32 rows: the packed weights are unpacked and their scales read per tile row).
+// 0.262 per MB.  A partly filled round is priced between its fullest CUs and the average one.  Fitted to the times of
+// every height and split at 119 launches (M 1-8192, N 1024-18432, K 1024-16384).  On 48 drawn launches of those
+// ranges, each timed with every height and split, the plan taken is on average 1.2 % (at most 10 %) from the fastest
+// one and takes half the time of 128-row tiles over the full reduction: 1 x 3072 x 12288 109.6 -> 15.5 us,
+// 333 x 3072 x 3072 30.9 -> 18.3, 768 x 6144 x 6144 68.9 -> 56.2, 1024 x 12288 -> 3072 108.4 -> 65.2.  From 2048 rows
+// the 128-row tiles are the faster ones (4096 x 3072 x 3072 53.5 against 59.6 and 73.9 for 64 and 32 rows: the packed
+// weights are unpacked and their scales read per tile row).
 W4Plan w4_plan(int64_t M, int64_t N, int64_t K, int cus, bool can_split) {
   struct Cost {
     int ib, wpc;
@@ -1613,11 +1614,11 @@ int launch_w4(W4Args p, void* ws, int64_t ws_bytes, hipStream_t st) {
 // A stage (128 reduction bytes) of a partly filled round is cheaper (less contention for L2 and HBM, and a higher
 // clock), and dearer the more of the staged bytes no other tile shares: its cost is scaled by (alpha + (1 - alpha)
 // fill) (1 + m unique), unique = the operands' rows over the rows that the tiles stage.  The constants are fitted
-// to the measured times of every shape and split at 552 launches (int8 and bf16, M 9-16896, outputs 512-32768,
-// reductions 512-32768), launches over 150 us with four times the weight; on 60 drawn launches beside those the plan
-// taken is on average 1.5 % from the fastest measured one and 8 % faster than the estimate it replaced, which was
-// fitted to full rounds (the 768-token input gradient to 16384 columns 196.6 -> 164.8 us, 512 x 6144 over 16384
-// 157.4 -> 114.0).
+// to the times of every shape and split at 552 launches (int8 and bf16, M 9-16896, outputs 512-32768, reductions
+// 512-32768), launches over 150 us with four times the weight.  On 72 launches drawn from M 9-16896 and widths
+// 512-16384, each timed with every shape and split, the plan taken is on average 1.6 % (at most 12 %) from the fastest
+// one, and 1.6 % faster than that of an estimate fitted to full rounds (bf16 768 x 16384 over 6144 195.8 -> 166.8 us,
+// int8 512 x 6144 over 16384 89.4 -> 75.7).
 struct SplitPlan {
   int64_t dp_tiles;   // tiles run over the full reduction
   int rem, s;         // remainder tiles and their pieces
@@ -1636,7 +1637,9 @@ constexpr TileCost TILE_COSTS[TILE_COUNT] = {
     {128, 128, 2, 0.722, 1.010, 3.243, 5.165},
 };
 
-// Shortest segmented reduction that is cut (stages).  Below it a launch takes under 60 us and a cut gains a few.
+// Shortest segmented reduction that is cut (stages).  It is not where a cut stops paying: on 40 launches below it (12-43
+// stages, M 17-2155) the cut that the estimate picks takes 0.79 of the uncut time on average (42 stages, 20 x 5120:
+// 26.5 against 15.0 us), and only under 15 stages is it slower (13 stages, 106 x 512: 9.2 against 10.3).
 constexpr int KSEG_SPLIT_MIN = 48;
 
 // The best plan of tile shape t for rows_a x rows_b outputs over nst stages.
