@@ -49,7 +49,7 @@ int k2q_check_device(void);
 
 /* (1) Rotate + per-row int8 quantize.
  * Replaces the point where Fp8Linear.forward receives x (reference quantize.py:48); the rotation and
- * the activation quantization have no reference code (north_star kernel (1)).  Also the int8 weight
+ * the activation quantization have no reference code.  Also the int8 weight
  * quantizer of Fp8Linear.__init__'s ConvRot counterpart (quantize.py:34-37): call it on W's rows.
  * x_rot (nullable) receives bf16(FWHT(x)/sqrt(128)). */
 int k2q_rotquant(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,

@@ -7,7 +7,7 @@ Reference interface followed (``quantize.py:23-68``): built from an existing ``n
 pages it (``mmdit.py:409-414``), and a walker that replaces the Linears of ``dit.blocks`` and returns the count
 (``quantize.py:54-68``).
 
-What differs is the arithmetic (BASELINE.json north_star): activations are rotated by a block Walsh-Hadamard
+What differs is the arithmetic: activations are rotated by a block Walsh-Hadamard
 transform and quantized per token to int8 on the fly; weights are stored rotated and quantized, int8 per output
 channel (``w8a8``) or packed int4 with one bf16 scale per 64-wide group (``w4a8``); the GEMM runs on int8
 MFMA with int32 accumulation.  All of it runs in the HIP library ``libk2q.so``; nothing here computes on the
