@@ -71,3 +71,43 @@ def test_fixup_ragged_equals_unsplit(k2, dev, M, N, K, r):
     assert torch.equal(y, L.gemm_w8a8(qx, sx, qw, sw, bias, u, B, 0.5, split=False))
     for t in ("256x256", "128x128"):
         assert torch.equal(y, L.gemm_w8a8(qx, sx, qw, sw, bias, u, B, 0.5, tile=t)), t
+
+
+@pytest.mark.parametrize("entry,M,N,K", [("GEMM_W8A8", 1024, 3072, 12288), ("GEMM_W8A8", 512, 6144, 16384),
+                                         ("GEMM_DX_LIN", 768, 16384, 6144), ("GEMM_DX_LIN", 130, 3072, 1024)])
+def test_the_plans_workspace_is_enough_and_less_is_left_alone(k2, dev, entry, M, N, K):
+    """The plan's bytes hold the pieces (what lies behind them stays as it was); with fewer the launch runs what it runs
+    without a workspace and writes nothing there."""
+    L = k2._lib
+    lib = L.load()
+    need = L.gemm_plan_ws_bytes(getattr(L, entry), M, N, K)
+    assert need > 0
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    st = torch.cuda.current_stream().cuda_stream
+    if entry == "GEMM_W8A8":
+        qx = torch.randint(-127, 128, (M, K), device=dev, dtype=torch.int8, generator=g)
+        qw = torch.randint(-127, 128, (N, K), device=dev, dtype=torch.int8, generator=g)
+        sx, sw = torch.rand(M, device=dev, generator=g), torch.rand(N, device=dev, generator=g)
+
+        def call(ws, nbytes):
+            y = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+            assert lib.k2q_gemm_w8a8(qx.data_ptr(), sx.data_ptr(), qw.data_ptr(), sw.data_ptr(), None, None, None, 0, 1.0,
+                                     M, N, K, y.data_ptr(), ws.data_ptr() if nbytes else None, nbytes, st) == 0
+            return y
+    else:
+        dy = torch.randn(M, N, device=dev, generator=g).bfloat16()
+        wt = torch.randn(K, N, device=dev, generator=g).bfloat16()
+
+        def call(ws, nbytes):
+            dx = torch.empty(M, K, device=dev, dtype=torch.bfloat16)
+            assert lib.k2q_gemm_dx_lin(dy.data_ptr(), wt.data_ptr(), M, N, K, None, None, 0, dx.data_ptr(),
+                                       ws.data_ptr() if nbytes else None, nbytes, st) == 0
+            return dx
+
+    ws = torch.full((need + 4096,), 0xA5, device=dev, dtype=torch.uint8)
+    whole = call(ws, 0)
+    assert torch.equal(call(ws, need - 16), whole) and bool((ws == 0xA5).all())
+    cut = call(ws, need)
+    assert bool((ws[need:] == 0xA5).all()) and not bool((ws[:need] == 0xA5).all())
+    assert torch.equal(cut, call(torch.empty(2 * need, device=dev, dtype=torch.uint8), 2 * need))
+    assert (cut.double() - whole.double()).norm() <= 2 ** -8 * whole.double().norm()    # at most a bf16 rounding apart
